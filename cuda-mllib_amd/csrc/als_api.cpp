@@ -273,6 +273,7 @@ struct cumf_handle {
 };
 
 namespace {
+  DevBuf stage;                   // packed factor rows on their way up or down (f not a multiple of 4)
 
 constexpr int kRmseBlocks = 1024;
 
@@ -325,6 +326,8 @@ int64_t bf16_stride(int f) {
 
 // Register budget of the launches without a tile table: two wavefronts
 // per SIMD while the accumulator tiles leave room for the solver's
+int ensure(DevBuf& b, size_t bytes) { return b.bytes >= bytes ? CUMF_OK : b.alloc(bytes); }
+
 // registers (up to 8 column blocks, f <= 124), one wavefront per SIMD
 // beyond (the two-wavefront build spills several hundred bytes per lane).
 int default_variant(int f) { return cumf::sweep_nb(f) >= 9 ? 1 : 2; }
@@ -674,9 +677,14 @@ int run_half_sweep(cumf_handle* h, int side, const Plan& p, const DevBuf& rowp, 
 }
 
 int upload_factors(cumf_handle* h, DevBuf& dst, DevBuf& dst_b, const float* src, int64_t rows) {
-  CUMF_HIP_TRY(hipMemsetAsync(dst.p, 0, dst.bytes, h->stream));
-  CUMF_HIP_TRY(hipMemcpy2DAsync(dst.p, sizeof(float) * h->ldf, src, sizeof(float) * h->f,
-                                sizeof(float) * h->f, rows, hipMemcpyHostToDevice, h->stream));
+  const size_t packed = sizeof(float) * (size_t)rows * h->f;
+  if (h->ldf == h->f) {
+    CUMF_HIP_TRY(hipMemcpyAsync(dst.p, src, packed, hipMemcpyHostToDevice, h->stream));
+  } else {
+    CUMF_TRY(ensure(h->stage, packed));
+    CUMF_HIP_TRY(hipMemcpyAsync(h->stage.p, src, packed, hipMemcpyHostToDevice, h->stream));
+    CUMF_HIP_TRY(cumf::launch_restride(h->stage.as<float>(), h->f, dst.as<float>(), h->ldf, rows, h->f, h->stream));
+  }
   if (h->opt.precision != CUMF_PREC_FP32)
     CUMF_HIP_TRY(cumf::launch_to_bf16(dst.as<float>(), h->ldf, dst_b.p, h->ldb, rows, h->f, h->stream));
   return CUMF_OK;
@@ -722,6 +730,9 @@ int cumf_create(int device, int f, float lambda, const cumf_options* opt, cumf_h
   if (o.cg_iters <= 0) o.cg_iters = kDefaultCgIters;
   if (o.cg_rounds <= 0) o.cg_rounds = kDefaultCgRounds;
   if (!(o.cg_tol > 0.f)) o.cg_tol = kDefaultCgTol;
+// The caller's packed rows go over in one flat copy and are laid out at the
+// factor stride on the device (and back in download_factors); where the
+// stride is f itself there is nothing to lay out.
   if (o.solver != CUMF_SOLVER_CHOLESKY && o.solver != CUMF_SOLVER_CG) {
     cumf::set_last_error("solver not built");
     return CUMF_ERR_UNSUPPORTED;
@@ -731,6 +742,18 @@ int cumf_create(int device, int f, float lambda, const cumf_options* opt, cumf_h
     return CUMF_ERR_INVALID;
   }
   if (o.warm_start < CUMF_WARM_PREV || o.warm_start > CUMF_WARM_BEST ||
+int download_factors(cumf_handle* h, const DevBuf& src, float* dst, int64_t rows) {
+  const size_t packed = sizeof(float) * (size_t)rows * h->f;
+  const void* from = src.p;
+  if (h->ldf != h->f) {
+    CUMF_TRY(ensure(h->stage, packed));
+    CUMF_HIP_TRY(cumf::launch_restride(src.as<float>(), h->ldf, h->stage.as<float>(), h->f, rows, h->f, h->stream));
+    from = h->stage.p;
+  }
+  CUMF_HIP_TRY(hipMemcpyAsync(dst, from, packed, hipMemcpyDeviceToHost, h->stream));
+  return CUMF_OK;
+}
+
       (o.warm_start != CUMF_WARM_PREV && o.solver != CUMF_SOLVER_CG)) {
     cumf::set_last_error("warm_start must be a CUMF_WARM_* value; only CUMF_SOLVER_CG has a start");
     return CUMF_ERR_INVALID;
@@ -965,12 +988,8 @@ int cumf_get_factors(cumf_handle* h, float* X, float* theta) {
     return CUMF_ERR_STATE;
   }
   DeviceGuard dg(h->device);
-  if (X)
-    CUMF_HIP_TRY(hipMemcpy2DAsync(X, sizeof(float) * h->f, h->X.p, sizeof(float) * h->ldf,
-                                  sizeof(float) * h->f, h->m, hipMemcpyDeviceToHost, h->stream));
-  if (theta)
-    CUMF_HIP_TRY(hipMemcpy2DAsync(theta, sizeof(float) * h->f, h->T.p, sizeof(float) * h->ldf,
-                                  sizeof(float) * h->f, h->n, hipMemcpyDeviceToHost, h->stream));
+  if (X) CUMF_TRY(download_factors(h, h->X, X, h->m));
+  if (theta) CUMF_TRY(download_factors(h, h->T, theta, h->n));
   CUMF_HIP_TRY(hipStreamSynchronize(h->stream));
   return CUMF_OK;
 }
@@ -1651,8 +1670,7 @@ int cumf_mlp_harvest(cumf_handle* h, cumf_mlp* mlp, int iters) {
     }
     rc = run_half_sweep(h, 0, h->plan_x, h->rp, h->ci, h->rv, h->T.as<float>(), h->X.as<float>(), h->Tb, h->Xb);
     if (rc != CUMF_OK) break;
-    if (hipMemcpy2DAsync(targets, sizeof(float) * h->f, h->X.p, sizeof(float) * h->ldf, sizeof(float) * h->f,
-                         h->m, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) {
+    if (cumf::launch_restride(h->X.as<float>(), h->ldf, targets, h->f, h->m, h->f, h->stream) != hipSuccess) {
       rc = CUMF_ERR_HIP;
       break;
     }
@@ -1850,8 +1868,6 @@ struct CacheLease {
     if (lk.owns_lock()) c = sc;
   }
 };
-
-int ensure(DevBuf& b, size_t bytes) { return b.bytes >= bytes ? CUMF_OK : b.alloc(bytes); }
 
 // Device-pointer half-sweep.  The CSR row pointers are read back to plan
 // the tasks (or to recognise the cached plan); factor buffers with

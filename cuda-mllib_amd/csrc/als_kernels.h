@@ -160,3 +160,6 @@ hipError_t launch_to_bf16(const float* src, int64_t ldf, void* dst, int64_t ldb,
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
 
 }  // namespace cumf
+// Device rows of `cols` floats, stride lds -> stride ldd (zero padded), ldd <= 4096.
+hipError_t launch_restride(const float* src, int64_t lds, float* dst, int64_t ldd, int64_t rows, int cols,
+                           hipStream_t s);

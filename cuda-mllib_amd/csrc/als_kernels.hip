@@ -113,6 +113,24 @@ __global__ __launch_bounds__(256) void to_bf16_kernel(const float* __restrict__ 
   }
 }
 
+// Rows of `cols` floats from stride lds to stride ldd, the columns past
+// `cols` written as zero (factors between the caller's packed layout and the
+// padded rows the sweeps read).  One pass at copy speed: a block takes whole
+// rows of about 8,192 destination floats, so the index division is 32 bits
+// wide.  It stands in for hipMemcpy2D, which moves pageable host memory row
+// by row (12,000 rows of 128 bytes: 20 ms up and 85 ms down; one flat copy
+// and this kernel: 0.1 ms) and for device rows needed a fill before it.
+__global__ __launch_bounds__(256) void restride_kernel(const float* __restrict__ src, int64_t lds,
+                                                       float* __restrict__ dst, int64_t ldd, int64_t rows, int cols,
+                                                       int block_rows) {
+  const int64_t r0 = (int64_t)blockIdx.x * block_rows;
+  const unsigned n = (unsigned)(rows - r0 < block_rows ? rows - r0 : block_rows), w = (unsigned)ldd;
+  for (unsigned i = threadIdx.x; i < n * w; i += 256) {
+    const unsigned r = i / w, c = i - r * w;
+    dst[(r0 + r) * ldd + c] = (int)c < cols ? src[(r0 + r) * lds + c] : 0.0f;
+  }
+}
+
 // One v_mfma_f32_16x16x32_bf16 with A[i][k] = i + k/32... (small integers,
 // exact in bf16) fed as lane l: A[l%16][8(l/16)+j]; writes the 64 x 4
 // result registers.  Pins the operand and result layout of the builtin.
@@ -201,6 +219,16 @@ hipError_t launch_to_bf16(const float* src, int64_t ldf, void* dst, int64_t ldb,
                           hipStream_t s) {
   if (rows <= 0) return hipSuccess;
   hipLaunchKernelGGL(to_bf16_kernel, dim3(2048), dim3(256), 0, s, src, ldf, (__bf16*)dst, ldb, rows, f);
+  return hipGetLastError();
+}
+
+hipError_t launch_restride(const float* src, int64_t lds, float* dst, int64_t ldd, int64_t rows, int cols,
+                           hipStream_t s) {
+  if (lds < cols || ldd < cols || ldd > 4096) return hipErrorInvalidValue;
+  if (rows <= 0) return hipSuccess;
+  const int64_t block_rows = (1024 + ldd - 1) / ldd;
+  hipLaunchKernelGGL(restride_kernel, dim3((unsigned)((rows + block_rows - 1) / block_rows)), dim3(256), 0, s, src,
+                     lds, dst, ldd, rows, cols, (int)block_rows);
   return hipGetLastError();
 }
 

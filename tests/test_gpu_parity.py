@@ -423,3 +423,22 @@ def test_bf16_gram_training_rmse_vs_fp64_oracle():
         h.iterate(iters)
         rm = h.rmse()
     assert abs(rm - hist[-1]) <= 1e-3, (rm, hist[-1])
+
+
+@pytest.mark.parametrize("f", [1, 3, 4, 10, 63, 100, 141, 255])
+@pytest.mark.parametrize("m,n", [(1, 1), (67, 3), (9001, 130)])
+def test_factors_round_trip_every_stride(f, m, n):
+    """Factors set on a handle come back bit for bit, whatever the padding of
+    the device rows (f a multiple of 4 or not), and again after a smaller and
+    a larger matrix through the same handle."""
+    rng = np.random.default_rng(f * 100003 + m)
+    with G.ALS(f, 0.05) as h:
+        for mm in (m, max(1, m // 2), m + 5):
+            rp = np.arange(mm + 1, dtype=np.int32)
+            h.set_ratings(mm, n, rp, rng.integers(0, n, mm), np.ones(mm, np.float32))
+            X = rng.standard_normal((mm, f)).astype(np.float32)
+            T = rng.standard_normal((n, f)).astype(np.float32)
+            h.set_factors(X=X, theta=T)
+            X2, T2 = h.get_factors()
+            np.testing.assert_array_equal(X2, X)
+            np.testing.assert_array_equal(T2, T)
