@@ -109,13 +109,37 @@ int plan_tasks(const int32_t* row_ptr, int64_t m, int split_, int f, std::vector
   return CUMF_OK;
 }
 
-// Wavefront task list of one rating matrix side on the device.
-struct Plan {
-  int64_t rows = 0, nnz = 0, ntasks = 0, nheavy = 0, nslots = 0;
+// The task list of whole rows, longest first, as the kernels above kMaxFusedF
+// divide it.
+struct LargeRanges {
+  int64_t ntasks = 0;
   int64_t light0 = 0;  // first task of at most kDualMaxRatingsHost ratings (tasks light0 .. ntasks-1)
   // Tasks [wg_t0[d], wg_t1[d]) have more than kDualMaxRatingsHost ratings
   // and d = (count + 16) / 16 <= kLargeDualWgMaxBlocks row blocks.
   int64_t wg_t0[cumf::kLargeDualWgMaxBlocks + 1] = {}, wg_t1[cumf::kLargeDualWgMaxBlocks + 1] = {};
+};
+
+// The same of a plan made on the device (lengths below 256 are classes of
+// their own there).
+LargeRanges large_ranges(const cumf::PlanSummary& p) {
+  LargeRanges r;
+  r.ntasks = p.ntasks;
+  // tasks of at least n ratings
+  auto at_least = [&](int n) -> int64_t { return n > 0 ? p.start[n - 1] : p.ntasks; };
+  r.light0 = at_least(cumf::kDualMaxRatingsHost + 1);
+  for (int d = 1; d <= cumf::kLargeDualWgMaxBlocks; ++d) {
+    const int lo = std::max(16 * (d - 1), cumf::kDualMaxRatingsHost + 1), hi = 16 * d - 1;
+    if (lo > hi) continue;
+    r.wg_t0[d] = at_least(hi + 1);
+    r.wg_t1[d] = at_least(lo);
+  }
+  return r;
+}
+
+// Wavefront task list of one rating matrix side on the device.
+struct Plan {
+  int64_t rows = 0, nnz = 0, ntasks = 0, nheavy = 0, nslots = 0;
+  LargeRanges large;
   int split = 0;
   int64_t bucket_t0[kBuckets] = {}, bucket_t1[kBuckets] = {};
   bool bucket_partial[kBuckets] = {};  // bucket b holds a split row's chunk
@@ -141,16 +165,16 @@ struct Plan {
       bucket_t1[b] = i + 1;
       bucket_partial[b] = bucket_partial[b] || t[(size_t)i].slot >= 0;
     }
-    light0 = ntasks;
+    large = LargeRanges{};
+    large.ntasks = large.light0 = ntasks;
     for (int b = 0; b < kBuckets && kBucketEdge[b + 1] <= cumf::kDualMaxRatingsHost + 1; ++b)
-      if (bucket_t1[b] > bucket_t0[b]) light0 = std::min(light0, bucket_t0[b]);
-    for (int d = 0; d <= cumf::kLargeDualWgMaxBlocks; ++d) wg_t0[d] = wg_t1[d] = 0;
+      if (bucket_t1[b] > bucket_t0[b]) large.light0 = std::min(large.light0, bucket_t0[b]);
     for (int64_t i = 0; i < ntasks; ++i) {
       const int cnt = t[(size_t)i].count;
       const int d = (cnt + 16) / 16;
       if (cnt <= cumf::kDualMaxRatingsHost || d > cumf::kLargeDualWgMaxBlocks) continue;
-      if (wg_t1[d] == 0) wg_t0[d] = i;
-      wg_t1[d] = i + 1;
+      if (large.wg_t1[d] == 0) large.wg_t0[d] = i;
+      large.wg_t1[d] = i + 1;
     }
     nheavy = (int64_t)hv.size();
     nslots = slots;
@@ -162,6 +186,32 @@ struct Plan {
     return CUMF_OK;
   }
 };
+
+// A plan made on the device for one call of the device entry points: the
+// buffers it works in are kept (at their largest so far) in the device's
+// cache and reused by the next call.
+struct DevicePlan {
+  DevBuf tasks, heavy, partial, work;
+  cumf::PlanSummary* summary = nullptr;  // pinned host memory the planner writes
+  DevicePlan() = default;
+  DevicePlan(const DevicePlan&) = delete;
+  DevicePlan& operator=(const DevicePlan&) = delete;
+  ~DevicePlan() {
+    if (summary) (void)hipHostFree(summary);
+  }
+};
+
+// Longest task of a matrix of nnz ratings: the caller's split size, less
+// where that would leave the chip waiting for one wavefront.  A task is at
+// most half of a wavefront's share when 2,048 of them (two per SIMD) run side
+// by side, and never under 2,048 ratings (a row of 2,048 costs a wavefront
+// about 0.1 ms at f = 100; finer cuts cost more in partial Grams than they
+// save).  Measured at 60,023 x 17,770, 12.4 million ratings, f = 50: the task
+// kernel 1.45 ms with a 16,384-rating task at its head; the whole call 0.85 ms
+// with 3,023.
+int adaptive_split(int split, int64_t nnz) {
+  return (int)std::min<int64_t>(split, std::max<int64_t>(2048, nnz / 4096));
+}
 
 int check_f(int f) {
   if (f < 1 || f > kMaxF) {
@@ -224,6 +274,7 @@ struct cumf_handle {
   int64_t ldb = 0;
   DevBuf tu, tv, tr;              // held-out COO
   DevBuf rmse_partial, rmse_out, fail;
+  DevBuf stage;                   // packed factor rows on their way up or down (f not a multiple of 4)
   Plan plan_x, plan_t;
   Timer timer;
   int64_t gram_flops = 0;
@@ -273,9 +324,10 @@ struct cumf_handle {
 };
 
 namespace {
-  DevBuf stage;                   // packed factor rows on their way up or down (f not a multiple of 4)
 
 constexpr int kRmseBlocks = 1024;
+
+int ensure(DevBuf& b, size_t bytes) { return b.bytes >= bytes ? CUMF_OK : b.alloc(bytes); }
 
 struct DeviceGuard {
   int prev = -1;
@@ -326,8 +378,6 @@ int64_t bf16_stride(int f) {
 
 // Register budget of the launches without a tile table: two wavefronts
 // per SIMD while the accumulator tiles leave room for the solver's
-int ensure(DevBuf& b, size_t bytes) { return b.bytes >= bytes ? CUMF_OK : b.alloc(bytes); }
-
 // registers (up to 8 column blocks, f <= 124), one wavefront per SIMD
 // beyond (the two-wavefront build spills several hundred bytes per lane).
 int default_variant(int f) { return cumf::sweep_nb(f) >= 9 ? 1 : 2; }
@@ -400,7 +450,7 @@ hipError_t bucket_launch(cumf_handle* h, int side, const Plan& p, const cumf::Sw
 //   * the rest: the work-group primal kernel.
 // Side by side when auxiliary streams are given (forked from s, joined
 // back); launches counts the kernel launches.
-hipError_t large_launches(const cumf::SweepArgs& a, const Plan& p, int* launches, hipStream_t s,
+hipError_t large_launches(const cumf::SweepArgs& a, const LargeRanges& p, int* launches, hipStream_t s,
                           hipStream_t aux0 = nullptr, hipStream_t aux1 = nullptr, hipEvent_t fork = nullptr,
                           hipEvent_t join0 = nullptr, hipEvent_t join1 = nullptr) {
   const bool dual = g_large_dual.load() != 0;
@@ -625,7 +675,7 @@ int run_half_sweep(cumf_handle* h, int side, const Plan& p, const DevBuf& rowp, 
     int nlaunch = 0;
     const size_t npend = h->timer.pending.size();
     CUMF_TRY(timed(h, Timer::TASK, [&] {
-      return large_launches(a, p, &nlaunch, h->stream, h->aux[0], h->aux[1], h->fork_ev, h->join_ev[0],
+      return large_launches(a, p.large, &nlaunch, h->stream, h->aux[0], h->aux[1], h->fork_ev, h->join_ev[0],
                             h->join_ev[1]);
     }));
     if (h->timer.pending.size() > npend) h->timer.pending.back().launches = std::max(1, nlaunch);
@@ -676,6 +726,9 @@ int run_half_sweep(cumf_handle* h, int side, const Plan& p, const DevBuf& rowp, 
   return CUMF_OK;
 }
 
+// The caller's packed rows go over in one flat copy and are laid out at the
+// factor stride on the device (and back in download_factors); where the
+// stride is f itself there is nothing to lay out.
 int upload_factors(cumf_handle* h, DevBuf& dst, DevBuf& dst_b, const float* src, int64_t rows) {
   const size_t packed = sizeof(float) * (size_t)rows * h->f;
   if (h->ldf == h->f) {
@@ -687,6 +740,18 @@ int upload_factors(cumf_handle* h, DevBuf& dst, DevBuf& dst_b, const float* src,
   }
   if (h->opt.precision != CUMF_PREC_FP32)
     CUMF_HIP_TRY(cumf::launch_to_bf16(dst.as<float>(), h->ldf, dst_b.p, h->ldb, rows, h->f, h->stream));
+  return CUMF_OK;
+}
+
+int download_factors(cumf_handle* h, const DevBuf& src, float* dst, int64_t rows) {
+  const size_t packed = sizeof(float) * (size_t)rows * h->f;
+  const void* from = src.p;
+  if (h->ldf != h->f) {
+    CUMF_TRY(ensure(h->stage, packed));
+    CUMF_HIP_TRY(cumf::launch_restride(src.as<float>(), h->ldf, h->stage.as<float>(), h->f, rows, h->f, h->stream));
+    from = h->stage.p;
+  }
+  CUMF_HIP_TRY(hipMemcpyAsync(dst, from, packed, hipMemcpyDeviceToHost, h->stream));
   return CUMF_OK;
 }
 
@@ -730,9 +795,6 @@ int cumf_create(int device, int f, float lambda, const cumf_options* opt, cumf_h
   if (o.cg_iters <= 0) o.cg_iters = kDefaultCgIters;
   if (o.cg_rounds <= 0) o.cg_rounds = kDefaultCgRounds;
   if (!(o.cg_tol > 0.f)) o.cg_tol = kDefaultCgTol;
-// The caller's packed rows go over in one flat copy and are laid out at the
-// factor stride on the device (and back in download_factors); where the
-// stride is f itself there is nothing to lay out.
   if (o.solver != CUMF_SOLVER_CHOLESKY && o.solver != CUMF_SOLVER_CG) {
     cumf::set_last_error("solver not built");
     return CUMF_ERR_UNSUPPORTED;
@@ -742,18 +804,6 @@ int cumf_create(int device, int f, float lambda, const cumf_options* opt, cumf_h
     return CUMF_ERR_INVALID;
   }
   if (o.warm_start < CUMF_WARM_PREV || o.warm_start > CUMF_WARM_BEST ||
-int download_factors(cumf_handle* h, const DevBuf& src, float* dst, int64_t rows) {
-  const size_t packed = sizeof(float) * (size_t)rows * h->f;
-  const void* from = src.p;
-  if (h->ldf != h->f) {
-    CUMF_TRY(ensure(h->stage, packed));
-    CUMF_HIP_TRY(cumf::launch_restride(src.as<float>(), h->ldf, h->stage.as<float>(), h->f, rows, h->f, h->stream));
-    from = h->stage.p;
-  }
-  CUMF_HIP_TRY(hipMemcpyAsync(dst, from, packed, hipMemcpyDeviceToHost, h->stream));
-  return CUMF_OK;
-}
-
       (o.warm_start != CUMF_WARM_PREV && o.solver != CUMF_SOLVER_CG)) {
     cumf::set_last_error("warm_start must be a CUMF_WARM_* value; only CUMF_SOLVER_CG has a start");
     return CUMF_ERR_INVALID;
@@ -1827,18 +1877,14 @@ int cumf_debug_copy(int device, int64_t bytes, int iters, double* ms_per_launch)
 
 namespace {
 
-// Per-device state the device-pointer half-sweep keeps between calls: the
-// task plan of the last rating matrix, reused when the next call brings the
-// same row pointers (Spark calls the drop-in once per half-sweep on the
-// same blocks), and device buffers kept at the largest size asked for so
-// far.  A call holds its device's cache for its whole duration; a
-// concurrent call on the same device that finds it held works with buffers
-// of its own.  The caches live until the process ends.
+// Per-device state the device-pointer half-sweep keeps between calls: device
+// buffers at the largest size asked for so far.  A call holds its device's
+// cache for its whole duration (it synchronises its stream before it gives it
+// back); a concurrent call on the same device that finds it held works with
+// buffers of its own.  The caches live until the process ends.
 struct SweepCache {
   std::mutex mu;
-  std::vector<int32_t> rp;  // row pointers the plan was built from
-  int f = 0, split = 0;
-  Plan plan;
+  DevicePlan plan;
   DevBuf theta, x, tpad, xpad, fail;
 };
 
@@ -1869,10 +1915,15 @@ struct CacheLease {
   }
 };
 
-// Device-pointer half-sweep.  The CSR row pointers are read back to plan
-// the tasks (or to recognise the cached plan); factor buffers with
-// f % 4 != 0 are re-strided through padded temporaries (the kernels read
-// factor rows with 16-byte loads).
+// Where the bound on a matrix's partial Grams is at most this, they are sized
+// by the bound and the sweep is launched behind the planner without waiting
+// for it; above it the host waits for the plan's counts (about 15 us).
+constexpr size_t kPartialBound = size_t(64) << 20;
+
+// Device-pointer half-sweep.  The tasks are planned on the device from the
+// row pointers (planner.hip); factor buffers with f % 4 != 0 are re-strided
+// through padded temporaries (the kernels read factor rows with 16-byte
+// loads).
 int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_t* d_col, const float* d_val,
                       const float* d_theta, float* d_x, int64_t m, int64_t n, int f, int64_t nnz, float lambda,
                       const cumf_options* opt, SweepCache* cache) {
@@ -1894,43 +1945,65 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
     cumf::set_last_error("compat_hermitian_bug is built for f <= " + std::to_string(kMaxFusedF));
     return CUMF_ERR_UNSUPPORTED;
   }
-  std::vector<int32_t> rp(m + 1);
-  CUMF_HIP_TRY(hipMemcpyAsync(rp.data(), d_row_ptr, sizeof(int32_t) * (m + 1), hipMemcpyDeviceToHost, stream));
-  CUMF_HIP_TRY(hipStreamSynchronize(stream));
-  if (rp[0] != 0 || rp[m] != nnz) {
-    cumf::set_last_error("row pointers must start at 0 and end at nnz");
+  DevicePlan local_plan;
+  DevBuf local_tpad, local_xpad, local_fail;
+  DevicePlan& plan = cache ? cache->plan : local_plan;
+  DevBuf* tpad = cache ? &cache->tpad : &local_tpad;
+  DevBuf* xpad = cache ? &cache->xpad : &local_xpad;
+  DevBuf* fail = cache ? &cache->fail : &local_fail;
+  const int64_t ldf = round_up4(f);
+  // Above kMaxFusedF whole rows are the tasks.
+  const int split = f <= kMaxFusedF ? adaptive_split(o.split, nnz) : INT_MAX;
+  const int64_t task_cap = m + nnz / split, heavy_cap = nnz / ((int64_t)split + 1);
+  const size_t slot_bytes = sizeof(float) * cumf::partial_floats_per_slot(f);
+  const int64_t slot_cap = heavy_cap + nnz / split;
+  if (task_cap > INT32_MAX) {
+    cumf::set_last_error("cumf_half_sweep_device: too many tasks");
     return CUMF_ERR_INVALID;
   }
-  Plan local_plan;
-  DevBuf local_tpad, local_xpad, local_fail;
-  Plan* plan = &local_plan;
-  DevBuf* tpad = &local_tpad;
-  DevBuf* xpad = &local_xpad;
-  DevBuf* fail = &local_fail;
-  if (cache) {
-    plan = &cache->plan;
-    tpad = &cache->tpad;
-    xpad = &cache->xpad;
-    fail = &cache->fail;
-    if (!(cache->f == f && cache->split == o.split && cache->rp == rp)) {
-      cache->rp.clear();  // no stale match if the build fails
-      CUMF_TRY(cache->plan.build(rp.data(), m, o.split, f));
-      cache->rp.swap(rp);
-      cache->f = f;
-      cache->split = o.split;
-    }
-  } else {
-    CUMF_TRY(local_plan.build(rp.data(), m, o.split, f));
+  CUMF_TRY(ensure(plan.tasks, sizeof(cumf::Task) * (size_t)task_cap));
+  CUMF_TRY(ensure(plan.heavy, sizeof(cumf::HeavyRow) * (size_t)heavy_cap));
+  CUMF_TRY(ensure(plan.work, cumf::plan_work_bytes()));
+  if (!plan.summary &&
+      hipHostMalloc(reinterpret_cast<void**>(&plan.summary), sizeof(cumf::PlanSummary), hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    plan.summary = nullptr;
+    cumf::set_last_error("hipHostMalloc of the plan summary failed");
+    return CUMF_ERR_NOMEM;
   }
-  const int64_t ldf = round_up4(f);
+  CUMF_HIP_TRY(cumf::launch_plan(d_row_ptr, m, nnz, split, plan.tasks.as<cumf::Task>(), task_cap,
+                                 plan.heavy.as<cumf::HeavyRow>(), heavy_cap, plan.work.p, plan.summary, stream));
+  // Refuses row pointers that do not start at 0, end at nnz and never
+  // decrease; with such a plan every task names no row, and nothing else of
+  // this call writes the result.
+  auto check_plan = [&]() -> int {
+    CUMF_HIP_TRY(hipStreamSynchronize(stream));
+    const cumf::PlanSummary& p = *plan.summary;
+    if (p.first != 0 || (int64_t)p.last != nnz) {
+      cumf::set_last_error("row pointers must start at 0 and end at nnz");
+      return CUMF_ERR_INVALID;
+    }
+    if (p.bad_row != INT_MAX) {
+      cumf::set_last_error("row pointers decrease at row " + std::to_string(p.bad_row));
+      return CUMF_ERR_INVALID;
+    }
+    return CUMF_OK;
+  };
+  const bool wait = f > kMaxFusedF || ldf != f || o.compat_hermitian_bug || slot_bytes * (size_t)slot_cap > kPartialBound;
+  int64_t ntasks = task_cap, nheavy = heavy_cap, nslots = slot_cap;
+  if (wait) {
+    CUMF_TRY(check_plan());
+    ntasks = plan.summary->ntasks;
+    nheavy = plan.summary->nheavy;
+    nslots = plan.summary->nslots;
+  }
+  if (!o.compat_hermitian_bug) CUMF_TRY(ensure(plan.partial, slot_bytes * (size_t)nslots));
   const float* theta = d_theta;
   float* x = d_x;
   if (ldf != f) {
     CUMF_TRY(ensure(*tpad, sizeof(float) * n * ldf));
     CUMF_TRY(ensure(*xpad, sizeof(float) * m * ldf));
-    CUMF_HIP_TRY(hipMemsetAsync(tpad->p, 0, sizeof(float) * n * ldf, stream));
-    CUMF_HIP_TRY(hipMemcpy2DAsync(tpad->p, sizeof(float) * ldf, d_theta, sizeof(float) * f,
-                                  sizeof(float) * f, n, hipMemcpyDeviceToDevice, stream));
+    CUMF_HIP_TRY(cumf::launch_restride(d_theta, f, tpad->as<float>(), ldf, n, f, stream));
     theta = tpad->as<float>();
     x = xpad->as<float>();
   }
@@ -1943,11 +2016,11 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
   a.theta = theta;
   a.x = x;
   a.ldf = ldf;
-  a.tasks = plan->tasks.as<cumf::Task>();
-  a.ntasks = plan->ntasks;
-  a.heavy = plan->heavy.as<cumf::HeavyRow>();
-  a.nheavy = plan->nheavy;
-  a.partial = plan->partial.as<float>();
+  a.tasks = plan.tasks.as<cumf::Task>();
+  a.ntasks = ntasks;
+  a.heavy = plan.heavy.as<cumf::HeavyRow>();
+  a.nheavy = nheavy;
+  a.partial = plan.partial.as<float>();
   a.fail_counter = fail->as<int>();
   a.f = f;
   a.lambda = lambda;
@@ -1967,14 +2040,14 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
   } else if (f > kMaxFusedF) {
     CUMF_HIP_TRY(cumf::prepare_large_kernel(f));
     int nlaunch = 0;
-    CUMF_HIP_TRY(large_launches(a, *plan, &nlaunch, stream));
+    CUMF_HIP_TRY(large_launches(a, large_ranges(*plan.summary), &nlaunch, stream));
   } else {
     CUMF_HIP_TRY(task_launch(a, default_variant(f), stream));
     CUMF_HIP_TRY(finish_launch(a, default_variant(f), stream));
   }
   if (ldf != f)
-    CUMF_HIP_TRY(hipMemcpy2DAsync(d_x, sizeof(float) * f, x, sizeof(float) * ldf, sizeof(float) * f, m,
-                                  hipMemcpyDeviceToDevice, stream));
+    CUMF_HIP_TRY(cumf::launch_restride(x, ldf, d_x, f, m, f, stream));
+  if (!wait) return check_plan();
   CUMF_HIP_TRY(hipStreamSynchronize(stream));
   return CUMF_OK;
 }

@@ -10,7 +10,7 @@ namespace cumf {
 // at rating index `start` of the CSR (absolute, so that no row-pointer load
 // precedes the first gather; rating indices fit int32 like the CSR's own).  slot < 0: the task covers the
 // whole row and solves it; slot >= 0: it writes a partial Gram to
-// partial[slot].
+// partial[slot].  row < 0: nothing to do (the tail of a list sized by a bound).
 struct Task {
   int32_t row;
   int32_t start;
@@ -18,7 +18,8 @@ struct Task {
   int32_t slot;
 };
 
-// A row whose Gram is the sum of `nchunks` partials starting at `slot`.
+// A row whose Gram is the sum of `nchunks` partials starting at `slot`
+// (row < 0: none).
 struct HeavyRow {
   int32_t row;
   int32_t slot;
@@ -81,6 +82,30 @@ struct SweepArgs {
 
 // Longest row the dual form takes (three staged chunks of 32 ratings).
 constexpr int kDualMaxRatingsHost = 95;
+
+// Length classes of the device planner (planner.hip): every length below 256
+// by itself, then eighths of an octave up to INT_MAX.
+constexpr int kPlanClasses = 256 + 8 * 23;
+__host__ __device__ inline int plan_class(int n) {
+  if (n < 256) return n;
+  const int e = 31 - __builtin_clz((unsigned)n);  // 8 .. 30
+  return 256 + 8 * (e - 8) + ((n >> (e - 3)) & 7);
+}
+// What the host needs of a plan made on the device.
+struct PlanSummary {
+  int32_t ntasks, nheavy, nslots;
+  int32_t bad_row;              // first row whose pointers decrease (INT_MAX: none)
+  int32_t first, last;          // row_ptr[0], row_ptr[m]
+  int32_t start[kPlanClasses];  // tasks of longer classes: where each class begins in the task list
+};
+size_t plan_work_bytes();
+// Plans m rows into tasks[0 .. task_cap) and heavy[0 .. heavy_cap), entries
+// past the plan naming row -1; with bad row pointers (see the summary) every
+// entry does.  task_cap >= m + nnz / split and heavy_cap >= nnz / (split + 1);
+// `work` holds plan_work_bytes() of device memory, `out` is host memory the
+// device can write, valid once the stream has passed.
+hipError_t launch_plan(const int32_t* row_ptr, int64_t m, int64_t nnz, int split, Task* tasks, int64_t task_cap,
+                       HeavyRow* heavy, int64_t heavy_cap, void* work, PlanSummary* out, hipStream_t s);
 
 // LDS of one CU, and the range of occupancy caps a launch accepts.
 constexpr int kLdsBytesPerCU = 160 * 1024;
@@ -157,9 +182,9 @@ hipError_t launch_mfma_layout(float* out, hipStream_t s);
 hipError_t launch_mfma_bf16_layout(float* out, hipStream_t s);
 hipError_t launch_to_bf16(const float* src, int64_t ldf, void* dst, int64_t ldb, int64_t rows, int f,
                           hipStream_t s);
-hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
-
-}  // namespace cumf
 // Device rows of `cols` floats, stride lds -> stride ldd (zero padded), ldd <= 4096.
 hipError_t launch_restride(const float* src, int64_t lds, float* dst, int64_t ldd, int64_t rows, int cols,
                            hipStream_t s);
+hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
+
+}  // namespace cumf

@@ -48,6 +48,7 @@ namespace CUMF_SNS {
 // row goes to scratch, or the row is solved.
 template <int NB, bool BF, bool CG>
 __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, float* lds, int lane) {
+  if (t.row < 0) return;
   float* xrow = a.x + (int64_t)t.row * a.ldf;
   __bf16* xb = BF ? reinterpret_cast<__bf16*>(a.x_b) + (int64_t)t.row * a.ldb : nullptr;
   if (t.count <= 0) {
@@ -119,6 +120,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
   extern __shared__ float lds[];
   const int lane = threadIdx.x;
   const HeavyRow h = a.heavy[blockIdx.x];
+  if (h.row < 0) return;
   f4 acc[num_tiles(NB)];
 #pragma unroll
   for (int i = 0; i < num_tiles(NB); ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};

@@ -106,7 +106,9 @@ typedef struct cumf_options {
   int32_t version;      /* CUMF_OPTIONS_VERSION */
   int32_t precision;    /* CUMF_PREC_* */
   int32_t split;        /* max ratings per wavefront task; longer rows are
-                           split and their partial Grams reduced (0: 16384) */
+                           split and their partial Grams reduced (0: 16384).
+                           The device entry points cut finer where a matrix
+                           is too small to fill the GPU with such tasks */
   int32_t timing;       /* 1: time every kernel launch with HIP events */
   int32_t use_graph;    /* 1: each half-sweep (X, Theta) is replayed from a
                            hipGraph captured at its first run; per-kernel
@@ -192,8 +194,10 @@ const char* cumf_last_error(void);
 
 /* Device-resident half-sweep with caller-owned device buffers (nothing
  * consumed, nothing copied): x (m x f) from theta (n x f) over the CSR.
- * Asynchronous on `stream`; the workspace it needs is allocated and freed
- * inside the call, which therefore synchronises `stream` before returning. */
+ * The tasks are planned on the device from the row pointers.  The workspace
+ * is kept per GPU between calls (at its largest so far), and the call
+ * synchronises `stream` before returning; calls that overlap on one GPU
+ * work with buffers of their own. */
 int cumf_half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_t* d_col,
                            const float* d_val, const float* d_theta, float* d_x, int64_t m,
                            int64_t n, int f, int64_t nnz, float lambda, const cumf_options* opt);
