@@ -58,14 +58,46 @@ __host__ __device__ constexpr int tile_index(int I, int J, int NB) {
   return I * NB - I * (I - 1) / 2 + (J - I);
 }
 
-// LDS floats per wave: the staging buffers of the Gram phase (FP32: two
-// chunks of NB tiles of 16 x 16 floats plus ratings; BF16: bf16_stage_bufs
+// Tile t of the upper triangle in tile_index order -> (I, J).
+__host__ __device__ constexpr int tile_row(int t, int NB) {
+  int I = 0;
+  while (t >= NB - I) {
+    t -= NB - I;
+    ++I;
+  }
+  return I;
+}
+__host__ __device__ constexpr int tile_col(int t, int NB) {
+  int I = 0;
+  while (t >= NB - I) {
+    t -= NB - I;
+    ++I;
+  }
+  return I + t;
+}
+
+template <typename F, int... qs>
+__device__ __forceinline__ void static_for_impl(F&& fn, std::integer_sequence<int, qs...>) {
+  (fn(std::integral_constant<int, qs>{}), ...);
+}
+// fn(std::integral_constant<int, q>) for q = 0 .. N-1, unrolled.
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& fn) {
+  static_for_impl(fn, std::make_integer_sequence<int, N>{});
+}
+
+// LDS floats per wave: the staging buffers of the Gram phase (FP32:
+// fp32_stage_bufs chunks of NB tiles of 16 x 16 floats plus ratings; BF16: bf16_stage_bufs
 // chunks of NB tiles of 32 x 16 bf16) and the buffers of the Cholesky solve (W blocks,
 // diagonal tile, identity, z, z2) share the same space.
 __host__ __device__ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 __host__ __device__ constexpr int chol_lds_floats(int NB) { return NB * 256 + 512 + 32 * NB; }
+// A staged FP32 chunk: NB tiles and 64 rating slots; four buffers where eight
+// wavefronts of them fit the CU's 160 KB (NB <= 4), else two.
+__host__ __device__ constexpr int fp32_chunk_floats(int NB) { return NB * 256 + 64; }
+__host__ __device__ constexpr int fp32_stage_bufs(int NB) { return 8 * 4 * 4 * fp32_chunk_floats(NB) <= 160 * 1024 ? 4 : 2; }
 __host__ __device__ constexpr int lds_floats_nb(int NB, bool bf) {
-  return cmax(bf ? bf16_stage_bufs(NB) * NB * 256 : 2 * NB * 256 + 2 * KB, chol_lds_floats(NB));
+  return cmax(bf ? bf16_stage_bufs(NB) * NB * 256 : fp32_stage_bufs(NB) * fp32_chunk_floats(NB), chol_lds_floats(NB));
 }
 
 
@@ -122,21 +154,126 @@ __device__ __forceinline__ void lds_order() {
 static __device__ const float kZeroRow[256] = {};
 
 // ---------------------------------------------------------------------------
+// FP32 products on the BF16 matrix pipe.  A float is the sum of three BF16
+// values h + m + l: h its upper half (truncated), m the remainder rounded to
+// BF16, l what is left, which is at most 8 bits and exact.  Of the nine
+// products of two such sums the six hh, hm, mh, mm, hl, lh carry the FP32
+// product to about 2^-24; ml, lm and ll are left out.  Six
+// v_mfma_f32_16x16x32_bf16 (16 cycles of the matrix pipe each) do 32 k-values
+// where eight v_mfma_f32_16x16x4_f32 take 32 cycles each.
+// ---------------------------------------------------------------------------
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  const uint32_t bx = __float_as_uint(x), by = __float_as_uint(y);
+  h = __builtin_amdgcn_perm(by, bx, 0x07060302);  // upper halves: y's above x's
+  const float rx = x - __uint_as_float(bx & 0xffff0000u), ry = y - __uint_as_float(by & 0xffff0000u);
+  m = __builtin_bit_cast(uint32_t, bf2{(__bf16)rx, (__bf16)ry});
+  const float lx = rx - __uint_as_float(m << 16), ly = ry - __uint_as_float(m & 0xffff0000u);
+  l = __builtin_amdgcn_perm(__float_as_uint(ly), __float_as_uint(lx), 0x07060302);
+}
+
+// The operands of one 16-column block for 32 k-values, eight to a lane, made
+// from two groups of four (HALF 0 and 1).
+struct Split8 {
+  u4 h, m, l;
+  template <int HALF>
+  __device__ __forceinline__ void set(float a, float b, float c, float d) {
+    uint32_t h0, m0, l0, h1, m1, l1;
+    split2(a, b, h0, m0, l0);
+    split2(c, d, h1, m1, l1);
+    h[2 * HALF] = h0;
+    h[2 * HALF + 1] = h1;
+    m[2 * HALF] = m0;
+    m[2 * HALF + 1] = m1;
+    l[2 * HALF] = l0;
+    l[2 * HALF + 1] = l1;
+  }
+  template <int HALF>
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int q = 2 * HALF; q < 2 * HALF + 2; ++q) h[q] = m[q] = l[q] = 0u;
+  }
+};
+// Product P = 0 .. 5 of the six, the small terms first.
+template <int P>
+__device__ __forceinline__ f4 split_mfma(const Split8& a, const Split8& b, f4 acc) {
+  static_assert(P >= 0 && P < 6, "six products");
+  const u4 av = P == 0 ? a.l : (P == 1 || P == 3 || P == 5) ? a.h : a.m;
+  const u4 bv = P == 1 ? b.l : (P == 0 || P == 4 || P == 5) ? b.h : b.m;
+  // 0: lh  1: hl  2: mm  3: hm  4: mh  5: hh
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av), __builtin_bit_cast(bf8, bv), acc, 0, 0, 0);
+}
+
+// acc[q] += the 32-rating (or 32-column) products of tile t = W + q STEP, for
+// every such tile of the upper triangle (FIRST: acc[q] = them).  A tile's six
+// products are summed from zero and added once, in FP32: one rounding at the
+// accumulator's size per 32 ratings where accumulating in place would take
+// six (and v_mfma_f32_16x16x4_f32 eight), so sums over long rows come out
+// nearer to the 64-bit ones than plain FP32 accumulation.  Four tiles at a
+// time, so that no product waits for the one before it.
+template <int NB, int W, int STEP, bool FIRST, int NQ>
+__device__ __forceinline__ void split_tiles(f4 (&acc)[NQ], const Split8 (&sp)[NB]) {
+  constexpr int NT = num_tiles(NB), G = 4;
+  static_for<(NQ + G - 1) / G>([&](auto gc) {
+    constexpr int q0 = decltype(gc)::value * G;
+    f4 t[G];
+    auto product = [&](auto pc) {
+      constexpr int P = decltype(pc)::value;
+      static_for<G>([&](auto kc) {
+        constexpr int k = decltype(kc)::value, q = q0 + k, tile = W + q * STEP;
+        if constexpr (q < NQ && tile < NT) {
+          constexpr int I = tile_row(tile, NB), J = tile_col(tile, NB);
+          t[k] = split_mfma<P>(sp[I], sp[J], P == 0 ? f4{0.f, 0.f, 0.f, 0.f} : t[k]);
+        }
+      });
+    };
+    static_for<6>(product);
+    static_for<G>([&](auto kc) {
+      constexpr int k = decltype(kc)::value, q = q0 + k, tile = W + q * STEP;
+      if constexpr (q < NQ && tile < NT) acc[q] = FIRST ? t[k] : acc[q] + t[k];
+    });
+  });
+}
+
+// Waits for this wave's outstanding LDS reads (a buffer they read may then be
+// overwritten by LDS-DMA); also a compiler memory barrier.
+__device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// ---------------------------------------------------------------------------
 // Gram of a contiguous range of one row's ratings (count >= 1): acc is set
 // to the range's augmented Gram, not added to.
 //
-// Staging: two LDS buffers per chunk of KB = 16 ratings, each NB tiles of
-// 16 rows x 16 floats (tile I holds columns 16I .. 16I+15 of the chunk's
-// factor rows, row stride 64 bytes), plus the KB ratings.  Load I of a
-// chunk fills tile I: lane l moves the 16 bytes of row l/4, columns
-// 16I + 4(l%4) .. +3, with global_load_lds_dwordx4 to byte 16l of the tile,
-// so every lane serves one fixed row of the chunk and loads that row's
-// column index itself (no cross-lane exchange).  sweep_nb(f) gives
-// 16 (NB-1) <= ldf < 16 NB: tiles 0 .. NB-2 lie inside the factor row, the
-// last tile holds the rest of it, the rating column (ldf) and padding.  In
-// the last tile, quads at or past ldf -- and every quad of a row past the
-// end of the range -- come from kZeroRow; the rating column is fed to the
-// MFMA from the rating buffer.  Gathers run one chunk ahead of the MFMAs.
+// Staging: LDS buffers of KB = 16 ratings each, NB tiles of 16 rows x 16
+// floats (tile I holds columns 16I .. 16I+15 of the chunk's factor rows, row
+// stride 64 bytes), plus the ratings.  Load I of a chunk fills tile I: lane l
+// moves the 16 bytes of row l/4, columns 16I + 4(l%4) .. +3, with
+// global_load_lds_dwordx4 to byte 16l of the tile, so every lane serves one
+// fixed row of the chunk and loads that row's column index itself (no
+// cross-lane exchange).  sweep_nb(f) gives 16 (NB-1) <= ldf < 16 NB: tiles
+// 0 .. NB-2 lie inside the factor row, the last tile holds the rest of it, the
+// rating column (ldf) and padding.  In the last tile, quads at or past ldf --
+// and every quad of a row past the end of the range, and its rating -- come
+// from kZeroRow; the rating column is fed to the MFMA from the rating buffer.
+//
+// A chunk goes from LDS to registers as split operands (half of a 32-rating
+// MFMA step), and its buffer is filled again at once, NBUF chunks ahead; the
+// matrix instructions of two chunks then run while those gathers are under
+// way.  Column indices are loaded NBUF chunks before their gather, in
+// registers that stay in place (the loop is unrolled NBUF times): an index is
+// as old as the chunk that is waited for, so using it waits for nothing newer.
+// Every chunk issues NB + 1 gathers, whatever its length, so the wait can
+// count them (index loads among them only make it stricter).
+//
+// Lane (g, c) supplies ratings g, 4 + g, 8 + g, 12 + g of a chunk for column c
+// (64 consecutive floats per LDS read).  What bounds it: at NB = 7, 32 ratings
+// are 168 matrix instructions of 16 cycles beside 308 VALU instructions of the
+// split, 112 additions and 56 LDS reads, against 224 matrix instructions of 32
+// cycles for plain FP32 ones.  Measured at 480,189 x 17,770, 99 million
+// ratings, f = 100, whole half-sweeps: Theta 13.7 -> 7.4 ms (40 GB of gathers,
+// 5.4 TB/s: now bound by them), X 16.5 -> 11.3 ms (now bound by its solves);
+// error against 64 bits 4.9e-6 -> 1.0e-6 and 1.2e-6 -> 5.4e-7.
 // ---------------------------------------------------------------------------
 template <int NB>
 __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32_t* __restrict__ col,
@@ -146,8 +283,9 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
                                            int lane) {
   const int g = lane >> 4, c = lane & 15;
   const int sr = lane >> 2, sq = lane & 3;  // staging row and quad of this lane
-  constexpr int CF = NB * 256;              // floats per staged chunk
-  float* rb = lds + 2 * CF;                 // ratings, [2][KB]
+  constexpr int CF = fp32_chunk_floats(NB);
+  constexpr int NBUF = fp32_stage_bufs(NB);
+  static_assert(NBUF % 2 == 0, "chunks are taken in pairs");
   const bool last_in = 16 * (NB - 1) + 4 * sq < (int)ldf;
   const bool rating_lane = 16 * (NB - 1) + c == (int)ldf;
   const int nch = (count + KB - 1) / KB;
@@ -155,55 +293,88 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
   // Column index of this lane's staging row in chunk ch (-1 past the end).
   auto load_ci = [&](int ch) -> int {
     const int k = ch * KB + sr;
-    return (ch < nch && k < count) ? col[start + k] : -1;
+    const int ci = col[start + (k < count ? k : count - 1)];
+    return k < count ? ci : -1;
   };
-  auto issue = [&](int ch, int ci) {
-    float* yb = lds + (ch & 1) * CF;
+  auto issue = [&](int ch, int buf, int ci) {
+    float* yb = lds + buf * CF;
     const float* rp = ci >= 0 ? theta + (int64_t)ci * ldf + 4 * sq : kZeroRow;
 #pragma unroll
     for (int I = 0; I < NB - 1; ++I)
       __builtin_amdgcn_global_load_lds(rp + 16 * I, (lds_void_t*)(yb + I * 256), 16, 0, 0);
-    const float* rl = last_in ? rp + 16 * (NB - 1) : kZeroRow;
+    const float* rl = (last_in && ci >= 0) ? rp + 16 * (NB - 1) : kZeroRow;
     __builtin_amdgcn_global_load_lds(rl, (lds_void_t*)(yb + (NB - 1) * 256), 16, 0, 0);
     const int k = ch * KB + lane;
-    if (lane < KB && k < count)
-      __builtin_amdgcn_global_load_lds(val + start + k, (lds_void_t*)(rb + (ch & 1) * KB), 4, 0, 0);
+    const float* vp = (lane < KB && k < count) ? val + start + k : kZeroRow;
+    __builtin_amdgcn_global_load_lds(vp, (lds_void_t*)(yb + NB * 256), 4, 0, 0);
   };
 
-  // The MFMAs of one staged chunk; the first chunk of the range starts the
-  // accumulators from zero (an inline-constant accumulator operand).
-  auto mfma_chunk = [&](const float* yb, const float* rr, int valid, auto first) {
+  Split8 sp[NB];
+  // A staged chunk into half HALF of the operands.
+  auto take = [&](const float* yb, auto half) {
+    constexpr int HALF = decltype(half)::value;
 #pragma unroll
-    for (int s = 0; s < KB / 4; ++s) {
-      const int row = 4 * s + g;
-      float a[NB];
+    for (int I = 0; I < NB; ++I) {
+      float v[4];
 #pragma unroll
-      for (int I = 0; I < NB; ++I) a[I] = yb[I * 256 + row * 16 + c];
-      if (rating_lane) a[NB - 1] = row < valid ? rr[row] : 0.0f;
+      for (int s = 0; s < 4; ++s) v[s] = yb[I * 256 + (4 * s + g) * 16 + c];
+      if (I == NB - 1) {
 #pragma unroll
-      for (int I = 0; I < NB; ++I)
-#pragma unroll
-        for (int J = I; J < NB; ++J)
-          acc[tile_index(I, J, NB)] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              a[I], a[J], (decltype(first)::value && s == 0) ? f4{0.f, 0.f, 0.f, 0.f} : acc[tile_index(I, J, NB)],
-              0, 0, 0);
+        for (int s = 0; s < 4; ++s) v[s] = rating_lane ? yb[NB * 256 + 4 * s + g] : v[s];
+      }
+      sp[I].template set<HALF>(v[0], v[1], v[2], v[3]);
     }
+    wait_lds_reads();
+  };
+  // The products of the two chunks in the operands.
+  auto mfmas = [&](auto first) {
+    split_tiles<NB, 0, 1, decltype(first)::value>(acc, sp);
   };
 
-  issue(0, load_ci(0));
-  int ci_next = load_ci(1);
-  for (int ch = 0; ch < nch; ++ch) {
-    wait_vm_all();  // chunk ch is in LDS; the column index of ch+1 is in ci_next
-    if (ch + 1 < nch) issue(ch + 1, ci_next);
-    ci_next = load_ci(ch + 2);
-    const float* yb = lds + (ch & 1) * CF;
-    const float* rr = rb + (ch & 1) * KB;
-    const int valid = count - ch * KB;
-    if (ch == 0) mfma_chunk(yb, rr, valid, std::true_type{});
-    else mfma_chunk(yb, rr, valid, std::false_type{});
-    lds_order();
+  int ahead[NBUF];  // column indices of the next chunk of each buffer
+  {
+    int now[NBUF];
+#pragma unroll
+    for (int d = 0; d < NBUF; ++d) now[d] = load_ci(d);
+#pragma unroll
+    for (int d = 0; d < NBUF; ++d) {
+      if (d < nch) issue(d, d, now[d]);
+      ahead[d] = load_ci(NBUF + d);
+      asm volatile("" ::: "memory");
+    }
+  }
+  for (int ch0 = 0; ch0 < nch; ch0 += NBUF) {
+    auto step = [&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      const int ch = ch0 + d;
+      // Chunk ch is in LDS once at most the gathers of the NBUF - 1 chunks
+      // after it are outstanding; near the end fewer were issued.
+      if (ch + NBUF - 1 < nch) wait_vm_recent<(NBUF - 1) * (NB + 1)>();
+      else wait_vm_all();
+      take(lds + d * CF, std::integral_constant<int, d & 1>{});
+      if (ch + NBUF < nch) issue(ch + NBUF, d, ahead[d]);
+      ahead[d] = load_ci(ch + 2 * NBUF);
+      asm volatile("" ::: "memory");
+    };
+    auto pair = [&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      if (ch0 + 2 * p < nch) {
+        step(std::integral_constant<int, 2 * p>{});
+        if (ch0 + 2 * p + 1 < nch) {
+          step(std::integral_constant<int, 2 * p + 1>{});
+        } else {
+#pragma unroll
+          for (int I = 0; I < NB; ++I) sp[I].template clear<1>();
+        }
+        if (p == 0 && ch0 == 0) mfmas(std::true_type{});
+        else mfmas(std::false_type{});
+      }
+    };
+    pair(std::integral_constant<int, 0>{});
+    if constexpr (NBUF == 4) pair(std::integral_constant<int, 1>{});
   }
   wait_vm_all();
+  lds_order();
 }
 
 // ---------------------------------------------------------------------------

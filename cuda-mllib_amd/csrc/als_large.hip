@@ -62,39 +62,12 @@ static_assert(kLargeDualMinBlocks == 7 && kLargeDualMaxBlocks == 16, "blocks 7 .
 
 __host__ __device__ constexpr int qmax(int NB) { return (num_tiles(NB) + 3) / 4; }
 
-template <typename F, int... qs>
-__device__ __forceinline__ void static_for_impl(F&& fn, std::integer_sequence<int, qs...>) {
-  (fn(std::integral_constant<int, qs>{}), ...);
-}
-// fn(std::integral_constant<int, q>) for q = 0 .. N-1, unrolled.
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& fn) {
-  static_for_impl(fn, std::make_integer_sequence<int, N>{});
-}
 // LDS floats: the tiles, then the diagonal-tile scratch, the identity, the
 // last block's W, z and x.  The Gram's staging (2 chunks of NB tiles and
 // their ratings) overlays the tile area.
 __host__ __device__ constexpr int large_lds_floats(int NB) { return num_tiles(NB) * 256 + 3 * 256 + 32 * NB; }
 // The dual form also keeps the row's ratings and column indices (256 each).
 __host__ __device__ constexpr int large_dual_wg_lds_floats(int NB) { return large_lds_floats(NB) + 512; }
-
-// Tile t of the upper triangle in tile_index order -> (I, J).
-__host__ __device__ constexpr int tile_row(int t, int NB) {
-  int I = 0;
-  while (t >= NB - I) {
-    t -= NB - I;
-    ++I;
-  }
-  return I;
-}
-__host__ __device__ constexpr int tile_col(int t, int NB) {
-  int I = 0;
-  while (t >= NB - I) {
-    t -= NB - I;
-    ++I;
-  }
-  return I + t;
-}
 
 // The Gram of wavefront W's tiles (t = W, W + 4, ...), left in acc, then
 // the ridge and the store of the tiles to their LDS slots.

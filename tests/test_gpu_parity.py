@@ -442,3 +442,59 @@ def test_factors_round_trip_every_stride(f, m, n):
             X2, T2 = h.get_factors()
             np.testing.assert_array_equal(X2, X)
             np.testing.assert_array_equal(T2, T)
+
+
+# One FP32 chunk is 16 ratings, two make a matrix step; four buffers up to
+# f = 60 (NB <= 4), two above; NB = 1 .. 9.
+@pytest.mark.parametrize("f", [4, 12, 27, 44, 60, 76, 92, 100, 120, 140])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -50, 2.0 ** 50])
+def test_fp32_gram_at_chunk_edges(f, scale):
+    """The FP32 Gram from split BF16 products against FP64, rating counts at
+    every edge of the staging and of the pairs, columns of mixed magnitude.
+    Bound per entry, in units of 2^-24 of the sum of the products' sizes: the
+    products left out (2^-24 each) and the summation inside a 32-rating step
+    (2 ulp = 2^-22 of its size per instruction that adds to the full value)
+    are below 8, and each step's addition costs one more.  Below FP32's normal
+    range (the smallest scale's smallest columns) a product's low parts may be
+    flushed: 2^-126 for each of its six."""
+    counts = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 79, 80, 81, 96, 97, 127, 128, 129, 257, 1000]
+    rng = np.random.default_rng(f)
+    n = 400
+    m = len(counts)
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ci = rng.integers(0, n, rp[-1]).astype(np.int32)
+    cv = rng.standard_normal(rp[-1]).astype(np.float32)
+    T = rng.standard_normal((n, f)) * np.exp2(rng.integers(-12, 13, (1, f))) * scale
+    T = T.astype(np.float32)
+    with G.ALS(f, 0.0) as h:
+        h.set_ratings(m, n, rp, ci, cv)
+        h.set_factors(theta=T)
+        got = h.row_gram(0, np.arange(m)).astype(np.float64)
+    bcol = (f + 3) // 4 * 4
+    for u, cnt in enumerate(counts):
+        Y = T[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+        r = cv[rp[u]:rp[u + 1]].astype(np.float64)
+        unit, low = 2.0 ** -24 * (8 + cnt / 32), 6 * cnt * 2.0 ** -126
+        for have, want, size in ((got[u][:f, :f], Y.T @ Y, np.abs(Y).T @ np.abs(Y)),
+                                 (got[u][:f, bcol], Y.T @ r, np.abs(Y).T @ np.abs(r))):
+            fits = size <= 2.0 ** 127  # (past FP32's range an entry is infinite, as any FP32 sum)
+            assert np.all(np.abs(have - want)[fits] <= (unit * size + low)[fits]), (f, cnt)
+
+
+def test_fp32_rows_with_infinities_and_nans_fail_alone():
+    """A factor that is not finite, or whose squares overflow, fails the rows
+    that read it (x = 0, counted) and no other."""
+    f, lam, n = 20, 0.05, 12
+    T = cumf.init_factors(n, f, 9)
+    T[0, 3], T[1, 5], T[2, 7], T[3, 0] = np.inf, -np.inf, np.nan, np.finfo(np.float32).max
+    ci = np.array([[0, 5, 6], [1, 5, 6], [2, 5, 6], [3, 5, 6], [4, 5, 6]], np.int32)
+    rp = np.arange(0, 16, 3, dtype=np.int32)
+    with G.ALS(f, lam) as h:
+        h.set_ratings(5, n, rp, ci.ravel(), np.full(15, 2.0, np.float32))
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 4
+    assert np.all(X[:4] == 0)
+    Xo, _ = O.half_sweep(np.array([0, 3], np.int32), ci[4], np.full(3, 2.0, np.float32), T, lam)
+    assert np.linalg.norm(X[4] - Xo[0]) <= 1e-5 * np.linalg.norm(Xo[0])
