@@ -6,14 +6,14 @@
 // arithmetic as the fused kernels (reference: als/src/cuda/als.cu:47-51,
 // 462-466 and 905-909 for the Gram and ridge, :1039-1054 for b, :935-997
 // for the solve):
-//   * Gram on MFMA (v_mfma_f32_16x16x4_f32): the NT = NB(NB+1)/2 upper
-//     tiles of the augmented [Y r]^T [Y r] are dealt round-robin to the
-//     four wavefronts (tile t to wavefront t % 4), which keep them in
-//     registers.  Chunks of 16 ratings are staged in LDS tile-major as in
-//     the fused kernels (tile I of a chunk gathered by wavefront I % 4 with
+//   * Gram on MFMA in FP32 from split BF16 products (als_device.h): the
+//     NT = NB(NB+1)/2 upper tiles of the augmented [Y r]^T [Y r] are dealt
+//     round-robin to the four wavefronts (tile t to wavefront t % 4), which
+//     keep them in registers.  32 ratings a step, staged in LDS tile-major as
+//     in the fused kernels (block I gathered by wavefront I % 4 with
 //     global_load_lds_dwordx4; the rating column written by the wavefront
-//     that gathers the last tile), double-buffered with one barrier per
-//     chunk.
+//     that gathers the last tile), split by the wavefront that gathered them
+//     and shared as MFMA operands through LDS.
 //   * The tiles then go to LDS (1 KB each, in accumulator order), and a
 //     blocked right-looking Cholesky runs on them with two barriers per
 //     16-column block K: the four wavefronts form the panel
@@ -31,13 +31,12 @@
 // row, als_large_dual_kernel): with Y the n x f matrix of the row's factor
 // rows and mu = lambda n, (Y^T Y + mu I)^{-1} Y^T r = Y^T (Y Y^T + mu I)^{-1} r,
 // so z solves the n x n system (Y Y^T + mu I) z = r and x = Y^T z:
-//   * K = Y Y^T in FP32 on v_mfma_f32_16x16x4_f32, straight from the factor
-//     rows: for each 16-column slab, lane (g, c) loads columns 4g .. 4g+3 of
-//     row 16I + c (16 bytes; the four lanes g of a row read 64 contiguous
-//     bytes) for every row block I, and the four columns feed four MFMA
-//     steps in which the same register is the A operand of block I and the
-//     B operand of block J = I.  The next slab's loads are issued before the
-//     current slab's MFMAs.
+//   * K = Y Y^T in FP32 from split BF16 products, straight from the factor
+//     rows: for each 32-column step, lane (g, c) loads columns 4g .. 4g+3 and
+//     16 + 4g .. 19 + 4g of row 16I + c (the four lanes g of a row read 64
+//     contiguous bytes) for every row block I; the split parts are the A
+//     operands of block I and the B operands of block J = I.  The next step's
+//     loads are issued before the current step's products.
 //   * r goes into column 16 NBD - 1 (past every live pivot), mu onto the
 //     first n diagonal entries, and the register-tile Cholesky of the fused
 //     kernels factors the NBD = (n + 16) / 16 <= 6 blocks and writes z to LDS.
@@ -63,37 +62,94 @@ static_assert(kLargeDualMinBlocks == 7 && kLargeDualMaxBlocks == 16, "blocks 7 .
 __host__ __device__ constexpr int qmax(int NB) { return (num_tiles(NB) + 3) / 4; }
 
 // LDS floats: the tiles, then the diagonal-tile scratch, the identity, the
-// last block's W, z and x.  The Gram's staging (2 chunks of NB tiles and
-// their ratings) overlays the tile area.
+// last block's W, z and x.  The Gram's operand buffers and staging overlay the
+// tile area.
 __host__ __device__ constexpr int large_lds_floats(int NB) { return num_tiles(NB) * 256 + 3 * 256 + 32 * NB; }
 // The dual form also keeps the row's ratings and column indices (256 each).
 __host__ __device__ constexpr int large_dual_wg_lds_floats(int NB) { return large_lds_floats(NB) + 512; }
 
-// The Gram of wavefront W's tiles (t = W, W + 4, ...), left in acc, then
-// the ridge and the store of the tiles to their LDS slots.
+// Operands of a 32-deep step in LDS, shared by the four wavefronts: per
+// 16-row block the parts h, m, l of the split floats (als_device.h), 16 bytes
+// a lane each.  A block is split once, by the wavefront that fetched it; split
+// by every wavefront for itself, the 17 blocks of f = 256 would cost more VALU
+// time than the products take on the matrix pipe.
+constexpr int kOpFloats = 3 * 256;  // per block
+__device__ __forceinline__ void write_op(float* ops, int I, const Split8& sp, int lane) {
+  u4* o = reinterpret_cast<u4*>(ops + I * kOpFloats) + lane;
+  o[0] = sp.h;
+  o[64] = sp.m;
+  o[128] = sp.l;
+}
+template <int NB>
+__device__ __forceinline__ void read_ops(const float* ops, Split8 (&sp)[NB], int lane) {
+#pragma unroll
+  for (int I = 0; I < NB; ++I) {
+    const u4* o = reinterpret_cast<const u4*>(ops + I * kOpFloats) + lane;
+    sp[I].h = o[0];
+    sp[I].m = o[64];
+    sp[I].l = o[128];
+  }
+}
+// Two operand buffers where they (and, in the primal form, the staging of a
+// step) fit the area that the tiles take over afterwards: one barrier a step
+// instead of two.
+__host__ __device__ constexpr bool op_double(int NB, bool dual) {
+  return (dual ? 6 : 8) * NB <= num_tiles(NB);
+}
+static_assert(3 * kLargeDualMinBlocks <= num_tiles(kLargeDualMinBlocks), "one operand buffer fits the tile area");
+static_assert(5 * 10 <= num_tiles(10), "an operand buffer and the staging fit the tile area");
+
+// The 32-deep steps of wavefront W's tiles (t = W, W + 4, ...): prep(step,
+// ops) puts this wavefront's blocks of a step into an operand buffer.
+template <int NB, int W, bool DB, typename P>
+__device__ __forceinline__ void op_steps(f4 (&acc)[qmax(NB)], int steps, float* lds, int lane, const P& prep) {
+#pragma unroll
+  for (int q = 0; q < qmax(NB); ++q) acc[q] = f4{0.f, 0.f, 0.f, 0.f};
+  prep(0, lds);
+  __syncthreads();  // step 0's operands are in LDS
+  for (int st = 0; st < steps; ++st) {
+    Split8 sp[NB];
+    read_ops<NB>(lds + (DB && (st & 1) ? NB * kOpFloats : 0), sp, lane);
+    if constexpr (DB) {
+      if (st + 1 < steps) prep(st + 1, lds + ((st & 1) ? 0 : NB * kOpFloats));
+    } else {
+      wait_lds_reads();
+      __syncthreads();  // every wavefront holds the step's operands: the buffer is free
+      if (st + 1 < steps) prep(st + 1, lds);
+    }
+    split_tiles<NB, W, 4, false>(acc, sp);
+    __syncthreads();  // the next step's operands are in LDS
+  }
+}
+
+// The Gram of wavefront W's tiles, left in acc, then the ridge and the store
+// of the tiles to their LDS slots.  A step is 32 ratings, staged as two groups
+// of 16 rows; wavefront W gathers, splits and shares the blocks I = W, W + 4,
+// ..., one step ahead of the products.
 template <int NB, int W>
 __device__ __forceinline__ void gram_tiles(const SweepArgs& a, int64_t start, int count, float* lds, int lane) {
   constexpr int NT = num_tiles(NB), Q = qmax(NB);
-  constexpr int CF = NB * 256;                // floats per staged chunk
+  constexpr bool DB = op_double(NB, false);
   constexpr bool WRITER = (NB - 1) % 4 == W;  // gathers the last tile, writes the ratings
+  float* stg = lds + (DB ? 2 : 1) * NB * kOpFloats;  // [2][NB] tiles; each wavefront reads only its own
   const int g = lane >> 4, c = lane & 15;
   const int sr = lane >> 2, sq = lane & 3;
   const int ldf = (int)a.ldf;
   const bool last_in = 16 * (NB - 1) + 4 * sq < ldf;
   const int rcol = ldf - 16 * (NB - 1);  // the rating's column in the last tile
-  const int nch = (count + KB - 1) / KB;
+  const int nst = (count + 2 * KB - 1) / (2 * KB);
   f4 acc[Q];
 
-  auto load_ci = [&](int ch) -> int {
-    const int k = ch * KB + sr;
-    return (ch < nch && k < count) ? a.col[start + k] : -1;
+  auto load_ci = [&](int st, int h) -> int {
+    const int k = 2 * KB * st + KB * h + sr;
+    return k < count ? a.col[start + k] : -1;
   };
-  auto load_r = [&](int ch) -> float {
-    const int k = ch * KB + lane;
-    return (lane < KB && ch < nch && k < count) ? a.val[start + k] : 0.0f;
+  auto load_r = [&](int st) -> float {
+    const int k = 2 * KB * st + lane;
+    return (lane < 2 * KB && k < count) ? a.val[start + k] : 0.0f;
   };
-  auto issue = [&](int ch, int ci) {
-    float* yb = lds + (ch & 1) * CF;
+  auto issue = [&](int h, int ci) {
+    float* yb = stg + h * NB * 256;
     const float* rp = ci >= 0 ? a.theta + (int64_t)ci * a.ldf + 4 * sq : kZeroRow;
 #pragma unroll
     for (int I = W; I < NB - 1; I += 4)
@@ -105,40 +161,42 @@ __device__ __forceinline__ void gram_tiles(const SweepArgs& a, int64_t start, in
       __builtin_amdgcn_global_load_lds(rl, (lds_void_t*)(yb + (NB - 1) * 256), 16, 0, 0);
     }
   };
-  auto mfma_chunk = [&](const float* yb, auto first) {
-#pragma unroll
-    for (int s = 0; s < KB / 4; ++s) {
-      const int row = 4 * s + g;
-      static_for<Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value, t = 4 * q + W;
-        if constexpr (t < NT) {
-          constexpr int I = tile_row(t, NB), J = tile_col(t, NB);
-          const float ai = yb[I * 256 + row * 16 + c], aj = yb[J * 256 + row * 16 + c];
-          acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              ai, aj, (decltype(first)::value && s == 0) ? f4{0.f, 0.f, 0.f, 0.f} : acc[q], 0, 0, 0);
-        }
-      });
-    }
-  };
 
+  issue(0, load_ci(0, 0));
+  issue(1, load_ci(0, 1));
   float rv = WRITER ? load_r(0) : 0.0f;
-  issue(0, load_ci(0));
-  int ci_next = load_ci(1);
-  for (int ch = 0; ch < nch; ++ch) {
-    wait_vm_all();  // this wavefront's gathers of chunk ch (and its rating loads) are done
-    const float* yb = lds + (ch & 1) * CF;
+  int ci0 = load_ci(1, 0), ci1 = load_ci(1, 1);
+  auto prep = [&](int st, float* ops) {
+    wait_vm_all();  // this wavefront's gathers of the step, its ratings and the next indices are there
     if constexpr (WRITER) {
-      if (lane < KB) lds[(ch & 1) * CF + (NB - 1) * 256 + lane * 16 + rcol] = rv;
+      if (lane < 2 * KB) stg[((lane >> 4) * NB + NB - 1) * 256 + (lane & 15) * 16 + rcol] = rv;
+      lds_order();
     }
-    __syncthreads();  // chunk ch staged by all; chunk ch-1 consumed by all
-    if (ch + 1 < nch) issue(ch + 1, ci_next);
-    ci_next = load_ci(ch + 2);
-    if constexpr (WRITER) rv = load_r(ch + 1);
-    if (ch == 0) mfma_chunk(yb, std::true_type{});
-    else mfma_chunk(yb, std::false_type{});
-  }
+    constexpr int M = (NB - W + 3) / 4;  // this wavefront's blocks
+    Split8 own[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+      float v[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[h][s] = stg[(h * NB + W + 4 * q) * 256 + (4 * s + g) * 16 + c];
+      own[q].template set<0>(v[0][0], v[0][1], v[0][2], v[0][3]);
+      own[q].template set<1>(v[1][0], v[1][1], v[1][2], v[1][3]);
+    }
+    wait_lds_reads();  // the staging may be filled again
+    if (st + 1 < nst) {
+      issue(0, ci0);
+      issue(1, ci1);
+    }
+    if constexpr (WRITER) rv = load_r(st + 1);
+    ci0 = load_ci(st + 2, 0);
+    ci1 = load_ci(st + 2, 1);
+#pragma unroll
+    for (int q = 0; q < M; ++q) write_op(ops, W + 4 * q, own[q], lane);
+  };
+  op_steps<NB, W, DB>(acc, nst, lds, lane, prep);
   wait_vm_all();
-  __syncthreads();  // every wavefront is done with the staging area
 
   const float ridge = a.lambda * (float)count;
   static_for<Q>([&](auto qc) {
@@ -156,55 +214,48 @@ __device__ __forceinline__ void gram_tiles(const SweepArgs& a, int64_t start, in
 }
 
 // Dual form on the work-group (rows of n <= 16 NB - 1 ratings):
-// wavefront W's tiles of K = Y Y^T (t = W, W + 4, ...), over 16-column
-// slabs of the factor rows listed in cs (lane (g, c) loads columns
-// 4g .. 4g+3 of row 16I + c of every row block I, the next slab's loads
-// issued before the current slab's MFMAs); then r into column 16 NB - 1,
-// mu = lambda n on the first n diagonal entries, and the store of the
-// tiles to their LDS slots.
+// wavefront W's tiles of K = Y Y^T (t = W, W + 4, ...), over 32-column steps
+// of the factor rows listed in cs.  Wavefront W loads the row blocks I = W,
+// W + 4, ... (lane (g, c): columns 4g .. 4g+3 and 16 + 4g .. 19 + 4g of the
+// step, row 16I + c), a step ahead of its split, and shares them; then r into
+// column 16 NB - 1, mu = lambda n on the first n diagonal entries, and the
+// store of the tiles to their LDS slots.
 template <int NB, int W>
 __device__ __forceinline__ void dual_tiles(const SweepArgs& a, int n, const int* cs, const float* rs, float* lds,
                                            int lane) {
-  constexpr int NT = num_tiles(NB), Q = qmax(NB);
+  constexpr int NT = num_tiles(NB), Q = qmax(NB), M = (NB - W + 3) / 4;
   const int g = lane >> 4, c = lane & 15;
   const int ldf = (int)a.ldf;
-  const int S = (ldf + 15) >> 4;  // 16-column slabs; columns past ldf are zero
-  const float* rp[NB];
+  const int steps = (ldf + 31) >> 5;  // columns past ldf are zero
+  const float* rp[M];
 #pragma unroll
-  for (int I = 0; I < NB; ++I) {
-    const int r = 16 * I + c;
-    rp[I] = r < n ? a.theta + (int64_t)cs[r] * ldf : kZeroRow;  // (kZeroRow holds 256 >= ldf floats)
+  for (int q = 0; q < M; ++q) {
+    const int r = 16 * (W + 4 * q) + c;
+    rp[q] = r < n ? a.theta + (int64_t)cs[r] * ldf : kZeroRow;  // (kZeroRow holds 256 >= ldf floats)
   }
-  auto load = [&](int sl, f4 (&v)[NB]) {
-    const int k = 16 * sl + 4 * g;
+  f4 v[M][2];
+  auto load = [&](int st) {
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
-      v[I] = k < ldf ? *reinterpret_cast<const f4*>(rp[I] + k) : f4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < 2; ++h) {
+      const int k = 32 * st + 16 * h + 4 * g;
+#pragma unroll
+      for (int q = 0; q < M; ++q)
+        v[q][h] = k < ldf ? *reinterpret_cast<const f4*>(rp[q] + k) : f4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  load(0);
+  auto prep = [&](int st, float* ops) {
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+      Split8 own;
+      own.template set<0>(v[q][0][0], v[q][0][1], v[q][0][2], v[q][0][3]);
+      own.template set<1>(v[q][1][0], v[q][1][1], v[q][1][2], v[q][1][3]);
+      write_op(ops, W + 4 * q, own, lane);
+    }
+    if (st + 1 < steps) load(st + 1);
   };
   f4 acc[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) acc[q] = f4{0.f, 0.f, 0.f, 0.f};
-  auto mfmas = [&](const f4 (&v)[NB]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      static_for<Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value, t = 4 * q + W;
-        if constexpr (t < NT) {
-          constexpr int I = tile_row(t, NB), J = tile_col(t, NB);
-          acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[I][j], v[J][j], acc[q], 0, 0, 0);
-        }
-      });
-  };
-  f4 va[NB], vb[NB];
-  load(0, va);
-  for (int sl = 0; sl < S; sl += 2) {
-    if (sl + 1 < S) load(sl + 1, vb);
-    mfmas(va);
-    if (sl + 1 < S) {
-      if (sl + 2 < S) load(sl + 2, va);
-      mfmas(vb);
-    }
-  }
+  op_steps<NB, W, op_double(NB, true)>(acc, steps, lds, lane, prep);
   const float ridge = a.lambda * (float)n;
   static_for<Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value, t = 4 * q + W;
@@ -259,11 +310,13 @@ __device__ __forceinline__ void diag_tile(float* slot, float* wdst, float* tsc, 
   if (last) *reinterpret_cast<f4*>(slot + 4 * lane) = *reinterpret_cast<const f4*>(tsc + 16 * c + 4 * g);
 }
 
+// Up to NB = 11 two work-groups' LDS fits a CU (70 KB each), so the registers
+// are held to two wavefronts per SIMD; above that a group has the CU to itself.
 // DUAL: the tasks are rows of n ratings, 16 (NB - 1) <= n <= 16 NB - 1,
 // solved in the dual form on NB row blocks (K = Y Y^T with r in column
 // 16 NB - 1, then x = Y^T z).
 template <int NB, bool DUAL>
-__global__ __launch_bounds__(kLT) __attribute__((amdgpu_waves_per_eu(1))) void als_large_kernel(SweepArgs a) {
+__global__ __launch_bounds__(kLT) __attribute__((amdgpu_waves_per_eu(NB <= 11 ? 2 : 1))) void als_large_kernel(SweepArgs a) {
   extern __shared__ float lds[];
   constexpr int NT = num_tiles(NB);
   // (the wavefront index is uniform: branches on it are scalar)
@@ -501,43 +554,39 @@ __device__ __forceinline__ bool large_dual_blocks(const SweepArgs& a, int n, con
                                                   float* lds, float* zs, int lane) {
   const int g = lane >> 4, c = lane & 15;
   const int ldf = (int)a.ldf;
-  const int S = (ldf + 15) >> 4;  // 16-column slabs; columns past ldf are zero
+  const int steps = (ldf + 31) >> 5;  // columns past ldf are zero
   const float* rp[NBD];
 #pragma unroll
   for (int I = 0; I < NBD; ++I) {
     const int r = 16 * I + c;
     rp[I] = r < n ? a.theta + (int64_t)cs[r] * ldf : kZeroRow;  // (kZeroRow holds 256 >= ldf floats)
   }
-  auto load = [&](int s, f4 (&v)[NBD]) {
-    const int k = 16 * s + 4 * g;
+  // 32-column steps: lane (g, c) loads columns 4g .. 4g+3 and 16 + 4g ..
+  // 19 + 4g of row 16I + c and splits them (als_device.h); the next step's
+  // loads are issued before the current step's products.
+  f4 v[NBD][2];
+  auto load = [&](int st) {
 #pragma unroll
-    for (int I = 0; I < NBD; ++I)
-      v[I] = k < ldf ? *reinterpret_cast<const f4*>(rp[I] + k) : f4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < 2; ++h) {
+      const int k = 32 * st + 16 * h + 4 * g;
+#pragma unroll
+      for (int I = 0; I < NBD; ++I)
+        v[I][h] = k < ldf ? *reinterpret_cast<const f4*>(rp[I] + k) : f4{0.f, 0.f, 0.f, 0.f};
+    }
   };
   f4 acc[num_tiles(NBD)];
 #pragma unroll
   for (int t = 0; t < num_tiles(NBD); ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  // Four MFMA steps per slab: in step j, lane (g, c) supplies column
-  // 16 s + 4 g + j of row 16 I + c, so every column enters each tile once.
-  auto mfmas = [&](const f4 (&v)[NBD]) {
+  load(0);
+  for (int st = 0; st < steps; ++st) {
+    Split8 sp[NBD];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int I = 0; I < NBD; ++I)
-#pragma unroll
-        for (int J = I; J < NBD; ++J)
-          acc[tile_index(I, J, NBD)] =
-              __builtin_amdgcn_mfma_f32_16x16x4f32(v[I][j], v[J][j], acc[tile_index(I, J, NBD)], 0, 0, 0);
-  };
-  f4 va[NBD], vb[NBD];
-  load(0, va);
-  for (int s = 0; s < S; s += 2) {
-    if (s + 1 < S) load(s + 1, vb);
-    mfmas(va);
-    if (s + 1 < S) {
-      if (s + 2 < S) load(s + 2, va);
-      mfmas(vb);
+    for (int I = 0; I < NBD; ++I) {
+      sp[I].template set<0>(v[I][0][0], v[I][0][1], v[I][0][2], v[I][0][3]);
+      sp[I].template set<1>(v[I][1][0], v[I][1][1], v[I][1][2], v[I][1][3]);
     }
+    if (st + 1 < steps) load(st + 1);
+    split_tiles<NBD, 0, 1, false>(acc, sp);
   }
   // r into column 16 NBD - 1 of the last block column (K is zero there:
   // rows past n are zero and 16 NBD - 1 >= n), mu on the diagonal.

@@ -171,3 +171,34 @@ def test_large_f_refuses_other_paths():
             h.autotune(reps=1)
     with pytest.raises(G.CumfError):
         G.ALS(257, 0.05)
+
+
+# f on both sides of the one / two operand-buffer line of the primal kernel
+# (f > 222) and of two work-groups per CU (f <= 172); counts at the edges of a
+# 32-rating step, of the wavefront dual form (95) and of every block count of
+# the work-group dual form (two operand buffers from 160 ratings on).
+@pytest.mark.parametrize("f", [141, 160, 172, 190, 222, 240, 256])
+def test_rows_at_every_step_and_block_edge(f):
+    """Relative residual of each row against the FP64 system on its factors,
+    at most 1e-5 (the plain path's bar)."""
+    counts = [1, 2, 15, 16, 31, 32, 33, 47, 63, 64, 65, 79, 94, 95, 96]
+    counts += [16 * d + e for d in range(7, 18) for e in (-1, 0, 1)] + [319, 320, 321, 1000, 2049]
+    lam, n = 0.05, 3000
+    rng = np.random.default_rng(f)
+    m = len(counts)
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ci = np.concatenate([rng.choice(n, c, replace=False) for c in counts]).astype(np.int32)
+    cv = rng.integers(1, 6, rp[-1]).astype(np.float32)
+    T = cumf.init_factors(n, f, 5)
+    with G.ALS(f, lam) as h:
+        h.set_ratings(m, n, rp, ci, cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 0
+    for u, cnt in enumerate(counts):
+        Y = T[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+        b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+        x = X[u].astype(np.float64)
+        res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(cnt)) * x
+        assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, cnt, np.linalg.norm(res) / np.linalg.norm(b))
