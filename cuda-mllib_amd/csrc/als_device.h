@@ -1914,4 +1914,122 @@ __device__ __forceinline__ void dual_solve_row_g(const SweepArgs& a, const Task&
   if (!ok && lane == 0) atomicAdd(a.fail_counter, 1);
 }
 
+// ---------------------------------------------------------------------------
+// The dual form on FP32 factors (any ldf <= 256), one wavefront per whole row
+// of n ratings, n + 1 <= 16 MB: K = Y Y^T straight from the factor rows (no
+// LDS staging), split products as in the FP32 Gram; then as above.
+// ---------------------------------------------------------------------------
+__host__ __device__ constexpr int fp32_dual_lds_floats(int MB) { return chol_lds_floats(MB) + 3 * 16 * MB; }
+
+// K = Y Y^T for the n rows listed in cs (n + 1 <= 16 NBD), r and the ridge
+// added, factored; z into zs.  False if a pivot was not positive and finite.
+template <int NBD>
+__device__ __forceinline__ bool fp32_dual_blocks(const SweepArgs& a, int n, const int* cs, const float* rs, float* lds,
+                                                 float* zs, int lane) {
+  const int g = lane >> 4, c = lane & 15;
+  const int ldf = (int)a.ldf;
+  const int steps = (ldf + 31) >> 5;  // columns past ldf are zero
+  const float* rp[NBD];
+#pragma unroll
+  for (int I = 0; I < NBD; ++I) {
+    const int r = 16 * I + c;
+    rp[I] = r < n ? a.theta + (int64_t)cs[r] * ldf : kZeroRow;  // (kZeroRow holds 256 >= ldf floats)
+  }
+  // 32-column steps: lane (g, c) loads columns 4g .. 4g+3 and 16 + 4g ..
+  // 19 + 4g of row 16I + c and splits them; the next step's loads are issued
+  // before the current step's products.
+  f4 v[NBD][2];
+  auto load = [&](int st) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = 32 * st + 16 * h + 4 * g;
+#pragma unroll
+      for (int I = 0; I < NBD; ++I)
+        v[I][h] = k < ldf ? *reinterpret_cast<const f4*>(rp[I] + k) : f4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  f4 acc[num_tiles(NBD)];
+#pragma unroll
+  for (int t = 0; t < num_tiles(NBD); ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  load(0);
+  for (int st = 0; st < steps; ++st) {
+    Split8 sp[NBD];
+#pragma unroll
+    for (int I = 0; I < NBD; ++I) {
+      sp[I].template set<0>(v[I][0][0], v[I][0][1], v[I][0][2], v[I][0][3]);
+      sp[I].template set<1>(v[I][1][0], v[I][1][1], v[I][1][2], v[I][1][3]);
+    }
+    if (st + 1 < steps) load(st + 1);
+    split_tiles<NBD, 0, 1, false>(acc, sp);
+  }
+  // r into column 16 NBD - 1 of the last block column (K is zero there:
+  // rows past n are zero and 16 NBD - 1 >= n), mu on the diagonal.
+#pragma unroll
+  for (int I = 0; I < NBD; ++I)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (c == 15) acc[tile_index(I, NBD - 1, NBD)][q] = rs[16 * I + 4 * g + q];
+  add_ridge<NBD>(acc, n, a.lambda * (float)n, lane);
+  return chol_solve<NBD>(acc, n, 16 * NBD - 1, lds, zs, 16 * NBD, lane);
+}
+
+// Row t (0 < t.count <= 16 MB - 1, a whole row).
+template <int MB>
+__device__ __forceinline__ void fp32_dual_row(const SweepArgs& a, const Task& t, float* lds, int lane) {
+  const int ldf = (int)a.ldf, n = t.count;
+  float* xrow = a.x + (int64_t)t.row * a.ldf;
+  float* zs = lds + chol_lds_floats(MB);
+  float* rs = zs + 16 * MB;
+  int* cs = reinterpret_cast<int*>(rs + 16 * MB);
+  for (int i = lane; i < 16 * MB; i += 64) {
+    const bool in = i < n;
+    rs[i] = in ? a.val[t.start + i] : 0.0f;
+    cs[i] = in ? a.col[t.start + i] : 0;
+  }
+  lds_order();
+  const int nbd = (n + 16) >> 4;  // blocks of the n x n system plus r's column
+  bool ok = false;
+  static_for<MB>([&](auto bc) {
+    constexpr int B = decltype(bc)::value + 1;
+    if (nbd == B) ok = fp32_dual_blocks<B>(a, n, cs, rs, lds, zs, lane);
+  });
+  lds_order();
+  // x = Y^T z (chol_solve left z = 0 if it failed): columns 4 lane .. +3.
+  const int k = 4 * lane;
+  if (k < ldf) {
+    f4 xv = {0.f, 0.f, 0.f, 0.f};
+    int i = 0;
+    for (; i + 4 <= n; i += 4) {
+      f4 y[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) y[q] = *reinterpret_cast<const f4*>(a.theta + (int64_t)cs[i + q] * ldf + k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float zq = zs[i + q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[e] = fmaf(zq, y[q][e], xv[e]);
+      }
+    }
+    for (; i < n; ++i) {
+      const f4 y = *reinterpret_cast<const f4*>(a.theta + (int64_t)cs[i] * ldf + k);
+      const float zq = zs[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xv[e] = fmaf(zq, y[e], xv[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xv[e] = (ok && k + e < a.f) ? xv[e] : 0.0f;
+    *reinterpret_cast<f4*>(xrow + k) = xv;
+  }
+  if (!ok && lane == 0) atomicAdd(a.fail_counter, 1);
+}
+
+// Row blocks of the dual system up to which the FP32 task kernel takes it in
+// place of the f x f system of NB blocks (0: never; 6: 95 ratings): wherever it
+// is the smaller one.  Measured, 480,189 x 17,770, f = 100, where 315,077 rows
+// have at most 95 ratings: X half-sweep 12.0 -> 10.1 ms; 60,023 x 17,770,
+// f = 128 3.4 -> 2.8 ms, f = 50 0.66 -> 0.65 ms.  A line one block lower gave
+// the same within 1%, two blocks lower 10.5 ms at f = 100 and 0.25 against
+// 0.22 ms at f = 32 (50 ratings a row).
+__host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB - 1 > 6 ? 6 : NB - 1; }
+
 }  // namespace cumf

@@ -539,123 +539,20 @@ __global__ __launch_bounds__(kLT) __attribute__((amdgpu_waves_per_eu(NB <= 11 ? 
   }
 }
 
-// Dual form: row blocks of the largest system (95 ratings plus r's column),
-// and the LDS floats of a row: the Cholesky's space for that many blocks,
-// then z, the ratings and the ratings' column indices (96 each).
+// One wavefront per task (a whole row of at most 95 ratings).
 constexpr int kLargeDualBlocks = (kDualMaxRatings + 16) / 16;
 static_assert(kLargeDualBlocks == 6, "six row blocks");
-__host__ __device__ constexpr int large_dual_lds_floats() { return chol_lds_floats(kLargeDualBlocks) + 3 * 96; }
-
-// K = Y Y^T for the n rows listed in cs (n + 1 <= 16 NBD), r and the ridge
-// added, factored; z into zs.  False if a pivot was not positive and
-// finite.
-template <int NBD>
-__device__ __forceinline__ bool large_dual_blocks(const SweepArgs& a, int n, const int* cs, const float* rs,
-                                                  float* lds, float* zs, int lane) {
-  const int g = lane >> 4, c = lane & 15;
-  const int ldf = (int)a.ldf;
-  const int steps = (ldf + 31) >> 5;  // columns past ldf are zero
-  const float* rp[NBD];
-#pragma unroll
-  for (int I = 0; I < NBD; ++I) {
-    const int r = 16 * I + c;
-    rp[I] = r < n ? a.theta + (int64_t)cs[r] * ldf : kZeroRow;  // (kZeroRow holds 256 >= ldf floats)
-  }
-  // 32-column steps: lane (g, c) loads columns 4g .. 4g+3 and 16 + 4g ..
-  // 19 + 4g of row 16I + c and splits them (als_device.h); the next step's
-  // loads are issued before the current step's products.
-  f4 v[NBD][2];
-  auto load = [&](int st) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int k = 32 * st + 16 * h + 4 * g;
-#pragma unroll
-      for (int I = 0; I < NBD; ++I)
-        v[I][h] = k < ldf ? *reinterpret_cast<const f4*>(rp[I] + k) : f4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  f4 acc[num_tiles(NBD)];
-#pragma unroll
-  for (int t = 0; t < num_tiles(NBD); ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  load(0);
-  for (int st = 0; st < steps; ++st) {
-    Split8 sp[NBD];
-#pragma unroll
-    for (int I = 0; I < NBD; ++I) {
-      sp[I].template set<0>(v[I][0][0], v[I][0][1], v[I][0][2], v[I][0][3]);
-      sp[I].template set<1>(v[I][1][0], v[I][1][1], v[I][1][2], v[I][1][3]);
-    }
-    if (st + 1 < steps) load(st + 1);
-    split_tiles<NBD, 0, 1, false>(acc, sp);
-  }
-  // r into column 16 NBD - 1 of the last block column (K is zero there:
-  // rows past n are zero and 16 NBD - 1 >= n), mu on the diagonal.
-#pragma unroll
-  for (int I = 0; I < NBD; ++I)
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (c == 15) acc[tile_index(I, NBD - 1, NBD)][q] = rs[16 * I + 4 * g + q];
-  add_ridge<NBD>(acc, n, a.lambda * (float)n, lane);
-  return chol_solve<NBD>(acc, n, 16 * NBD - 1, lds, zs, 16 * NBD, lane);
-}
-
-// One wavefront per task (a whole row of at most 95 ratings).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void als_large_dual_kernel(SweepArgs a) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x;
   const Task t = a.tasks[blockIdx.x];
-  const int ldf = (int)a.ldf;
-  float* xrow = a.x + (int64_t)t.row * a.ldf;
-  const int n = t.count;
-  if (n <= 0 || n > kDualMaxRatings) {  // (the host launches only rows that fit)
-    for (int i = lane; i < ldf; i += 64) xrow[i] = 0.0f;
-    if (n > 0 && lane == 0) atomicAdd(a.fail_counter, 1);
+  if (t.count <= 0 || t.count > kDualMaxRatings) {  // (the host launches only rows that fit)
+    float* xrow = a.x + (int64_t)t.row * a.ldf;
+    for (int i = lane; i < (int)a.ldf; i += 64) xrow[i] = 0.0f;
+    if (t.count > 0 && lane == 0) atomicAdd(a.fail_counter, 1);
     return;
   }
-  float* zs = lds + chol_lds_floats(kLargeDualBlocks);
-  float* rs = zs + 96;
-  int* cs = reinterpret_cast<int*>(rs + 96);
-  for (int i = lane; i < 96; i += 64) {
-    const bool in = i < n;
-    rs[i] = in ? a.val[t.start + i] : 0.0f;
-    cs[i] = in ? a.col[t.start + i] : 0;
-  }
-  lds_order();
-  const int nbd = (n + 16) >> 4;  // blocks of the n x n system plus r's column
-  bool ok;
-  if (nbd == 1) ok = large_dual_blocks<1>(a, n, cs, rs, lds, zs, lane);
-  else if (nbd == 2) ok = large_dual_blocks<2>(a, n, cs, rs, lds, zs, lane);
-  else if (nbd == 3) ok = large_dual_blocks<3>(a, n, cs, rs, lds, zs, lane);
-  else if (nbd == 4) ok = large_dual_blocks<4>(a, n, cs, rs, lds, zs, lane);
-  else if (nbd == 5) ok = large_dual_blocks<5>(a, n, cs, rs, lds, zs, lane);
-  else ok = large_dual_blocks<6>(a, n, cs, rs, lds, zs, lane);
-  lds_order();
-  // x = Y^T z (chol_solve left z = 0 if it failed): columns 4 lane .. +3.
-  const int k = 4 * lane;
-  if (k >= ldf) return;
-  f4 xv = {0.f, 0.f, 0.f, 0.f};
-  int i = 0;
-  for (; i + 4 <= n; i += 4) {
-    f4 y[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) y[q] = *reinterpret_cast<const f4*>(a.theta + (int64_t)cs[i + q] * ldf + k);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float zq = zs[i + q];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) xv[e] = fmaf(zq, y[q][e], xv[e]);
-    }
-  }
-  for (; i < n; ++i) {
-    const f4 y = *reinterpret_cast<const f4*>(a.theta + (int64_t)cs[i] * ldf + k);
-    const float zq = zs[i];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) xv[e] = fmaf(zq, y[e], xv[e]);
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) xv[e] = (ok && k + e < a.f) ? xv[e] : 0.0f;
-  *reinterpret_cast<f4*>(xrow + k) = xv;
-  if (!ok && lane == 0) atomicAdd(a.fail_counter, 1);
+  fp32_dual_row<kLargeDualBlocks>(a, t, lds, lane);
 }
 
 template <int NB, bool DUAL>
@@ -704,7 +601,7 @@ hipError_t launch_large_dual_kernel(const SweepArgs& a, int64_t ntasks, hipStrea
     return hipErrorInvalidValue;
   if (ntasks == 0) return hipSuccess;
   hipLaunchKernelGGL(als_large_dual_kernel, dim3((unsigned)ntasks), dim3(64),
-                     sizeof(float) * large_dual_lds_floats(), s, a);
+                     sizeof(float) * fp32_dual_lds_floats(kLargeDualBlocks), s, a);
   return hipGetLastError();
 }
 

@@ -64,6 +64,12 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
     return;
   }
 
+  if constexpr (!BF && !CG && fp32_dual_max_blocks(NB) > 0) {
+    if (t.slot < 0 && t.count <= 16 * fp32_dual_max_blocks(NB) - 1) {
+      fp32_dual_row<fp32_dual_max_blocks(NB)>(a, t, lds, lane);
+      return;
+    }
+  }
   // The row's current factor (the CG start) is fetched before the Gram so
   // that its latency hides behind the gathers.
   float xpre[rows_per_lane(NB)];
@@ -159,6 +165,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
       const int64_t s = a.row_ptr[row];
       const int cnt = a.row_ptr[row + 1] - a.row_ptr[row];
       lds_order();
+      if constexpr (!BF && fp32_dual_max_blocks(NB) > 0) {  // as the task kernel solves them
+        if (cnt > 0 && cnt <= 16 * fp32_dual_max_blocks(NB) - 1) {
+          fp32_dual_row<fp32_dual_max_blocks(NB)>(a, Task{(int32_t)row, (int32_t)s, cnt, -1}, lds, lane);
+          continue;
+        }
+      }
       if (cnt > 0) gram_any<NB, BF>(acc, a, s, cnt, lds, lane);
     } else {
       const HeavyRow h = a.heavy[-1 - e];
@@ -220,6 +232,7 @@ static hipError_t launch_nb(const SweepArgs& a, hipStream_t s, int which) {
   constexpr bool CG = CUMF_SWEEP_SOLVER == 1;
   const bool bf = a.precision != 0;
   size_t shmem = sizeof(float) * (size_t)cmax(lds_floats_nb(NB, bf), CG ? cg_lds_floats(NB, a.f) : 0);
+  static_assert(fp32_dual_lds_floats(fp32_dual_max_blocks(NB)) <= lds_floats_nb(NB, false), "the dual form's space");
   if (which == 0 && a.persistent == 0 && a.occupancy > 0) {
     if (a.occupancy < kMinOccupancy || a.occupancy > kMaxOccupancy) return hipErrorInvalidValue;
     if (occupancy_lds_bytes(a.occupancy) > shmem) shmem = occupancy_lds_bytes(a.occupancy);

@@ -498,3 +498,31 @@ def test_fp32_rows_with_infinities_and_nans_fail_alone():
     assert np.all(X[:4] == 0)
     Xo, _ = O.half_sweep(np.array([0, 3], np.int32), ci[4], np.full(3, 2.0, np.float32), T, lam)
     assert np.linalg.norm(X[4] - Xo[0]) <= 1e-5 * np.linalg.norm(Xo[0])
+
+
+@pytest.mark.parametrize("f", [12, 32, 50, 76, 92, 100, 128, 140])
+def test_short_rows_on_both_sides_of_the_dual_line(f):
+    """FP32 rows whose n x n system is smaller than the f x f one are solved in
+    it; every length up to 97 and both sides of each block edge, against the
+    FP64 system on the same factors: relative residual at most 1e-5."""
+    lam, n = 0.05, 700
+    rng = np.random.default_rng(f)
+    counts = np.arange(0, 114)
+    m = len(counts)
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ci = np.concatenate([rng.choice(n, c, replace=False) for c in counts]).astype(np.int32)
+    cv = rng.standard_normal(rp[-1]).astype(np.float32) * 3
+    T = cumf.init_factors(n, f, 5)
+    with G.ALS(f, lam) as h:
+        h.set_ratings(m, n, rp, ci, cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 0
+    assert np.all(X[0] == 0)
+    for u in range(1, m):
+        Y = T[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+        b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+        x = X[u].astype(np.float64)
+        res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(counts[u])) * x
+        assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, u, np.linalg.norm(res) / np.linalg.norm(b))
