@@ -67,6 +67,8 @@ struct SweepArgs {
   int* fb_count;
   // persistent > 0: launch that many wavefronts, each taking tasks from
   // *task_counter (zero before the launch) until ntasks are taken.
+  // launch_rows_kernel: that many work-groups over the rows 0 .. ntasks of
+  // row_ptr; task_counter[0] and [2] zero before the launch.
   int persistent;
   int* task_counter;
   // occupancy > 0 (one-task-per-group launches): at most that many
@@ -141,13 +143,15 @@ hipError_t launch_fallback_reset(int* count, int n, hipStream_t s);
 // Launchers of the sweep kernels, per register budget (w1, w2) and solver
 // family (chol: Cholesky task/finish kernels and the CG path's fallback;
 // cg: CG task/finish kernels; chol also holds the dual-form task kernel
-// for rows of at most 95 ratings, BF16 factors only).
+// for rows of at most 95 ratings, BF16 factors only, and the kernel over
+// whole rows without a plan, FP32 only).
 #define CUMF_SWEEP_LAUNCHERS                                                \
   namespace chol {                                                          \
   hipError_t launch_task_kernel(const SweepArgs& a, hipStream_t s);         \
   hipError_t launch_finish_kernel(const SweepArgs& a, hipStream_t s);       \
   hipError_t launch_fallback_kernel(const SweepArgs& a, hipStream_t s);     \
   hipError_t launch_dual_kernel(const SweepArgs& a, hipStream_t s);         \
+  hipError_t launch_rows_kernel(const SweepArgs& a, hipStream_t s);         \
   }                                                                         \
   namespace cg {                                                            \
   hipError_t launch_task_kernel(const SweepArgs& a, hipStream_t s);         \

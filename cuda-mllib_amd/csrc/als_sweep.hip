@@ -97,8 +97,7 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
 }
 
 // tasks[0 .. ntasks): one work-group per task, or (PERSISTENT) a grid of
-// wavefronts that take tasks from a counter until none are left (with no
-// task list, PERSISTENT takes the rows 0 .. ntasks themselves).  Separate
+// wavefronts that take tasks from a counter until none are left.  Separate
 // instantiations: the loop changes register allocation (more spill), so the
 // one-task-per-group kernel keeps its own.
 template <int NB, bool BF, bool CG, bool PERSISTENT>
@@ -114,9 +113,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
       idx = __builtin_amdgcn_readfirstlane(idx);
       if (idx >= a.ntasks) break;
       lds_order();
-      // Without a task list the tasks are the rows themselves, whole.
-      const Task t = a.tasks ? a.tasks[idx] : Task{idx, a.row_ptr[idx], a.row_ptr[idx + 1] - a.row_ptr[idx], -1};
-      run_task<NB, BF, CG>(a, t, lds, lane);
+      run_task<NB, BF, CG>(a, a.tasks[idx], lds, lane);
     }
   }
 }
@@ -225,6 +222,89 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
 }
 #endif
 
+#if CUMF_SWEEP_SOLVER == 0
+// The rows 0 .. ntasks themselves, FP32, without a task list, plan or scratch
+// memory: one work-group per CU, two passes.
+//   * Rows of more than kLongRow ratings are solved by the work-group
+//     together: each wavefront forms the Gram of its share of the ratings, the
+//     shares are added through LDS in wavefront order, and wavefront 0 solves.
+//     The groups take batches of rows from a counter to look for them.  By
+//     itself a wavefront needs 0.84 ms for a row of 15,136 ratings at f = 64,
+//     which was all of a 2,048-row call; the call now takes 0.19 ms.
+//   * The other rows go to the wavefronts one by one, from a second counter,
+//     solved as the task kernel solves them (the device entry points with a
+//     plan do not split rows up to kLongRow ratings either).
+constexpr int kRowsWaves = 4 * CUMF_TASK_WAVES;  // wavefronts per group: all a CU holds
+constexpr int kLongRow = 2048;
+
+template <int NB>
+__global__ __launch_bounds__(64 * kRowsWaves)
+__attribute__((amdgpu_waves_per_eu(CUMF_TASK_WAVES))) void als_rows_kernel(SweepArgs a, int batch) {
+  constexpr int WF = lds_floats_nb(NB, false), NT = num_tiles(NB);
+  static_assert(NT * 256 <= kRowsWaves * WF, "a Gram fits the wavefronts' staging");
+  __shared__ __align__(16) float lds_all[kRowsWaves * WF];
+  __shared__ int next;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* lds = lds_all + wv * WF;
+  // (The first batch, and below the first row, is this group's by its place
+  // in the grid: some 2,000 adds to one counter at the start of the kernel
+  // would take longer than a small call.)
+  for (int64_t b = blockIdx.x;;) {
+    const int64_t u0 = b * batch;
+    if (u0 >= a.ntasks) break;
+    const int64_t mine = u0 + lane;
+    const bool is_long = lane < batch && mine < a.ntasks && a.row_ptr[mine + 1] - a.row_ptr[mine] > kLongRow;
+    for (uint64_t todo = __ballot(is_long); todo; todo &= todo - 1) {
+      const int64_t u = u0 + __builtin_ctzll(todo);
+      const int start = a.row_ptr[u], n = a.row_ptr[u + 1] - start;
+      // Shares of whole 32-rating steps.
+      const int share = ((n + 31) / 32 + kRowsWaves - 1) / kRowsWaves * 32;
+      const int off = wv * share, cnt = n - off < share ? n - off : share;
+      f4 acc[NT];
+      if (cnt > 0) {
+        gram_any<NB, false>(acc, a, (int64_t)start + off, cnt, lds, lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
+      }
+      __syncthreads();  // every share is formed: the staging is free
+      for (int w = 1; w < kRowsWaves; ++w) {
+        if (wv == w) {
+#pragma unroll
+          for (int i = 0; i < NT; ++i) *reinterpret_cast<f4*>(lds_all + i * 256 + 4 * lane) = acc[i];
+        }
+        __syncthreads();
+        if (wv == 0) {
+#pragma unroll
+          for (int i = 0; i < NT; ++i) acc[i] += *reinterpret_cast<const f4*>(lds_all + i * 256 + 4 * lane);
+        }
+        __syncthreads();
+      }
+      if (wv == 0) {
+        add_ridge<NB>(acc, a.f, a.lambda * (float)n, lane);
+        solve_row<NB, false>(acc, a, false, lds, u, nullptr, lane, 0);
+        lds_order();
+      }
+    }
+    if ((int64_t)gridDim.x * batch >= a.ntasks) break;  // (every batch had its group)
+    __syncthreads();  // `next` has been read by all
+    if (threadIdx.x == 0) next = atomicAdd(a.task_counter + 2, 1);
+    __syncthreads();
+    b = (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane(next);
+  }
+  const int64_t waves = (int64_t)gridDim.x * kRowsWaves;
+  for (int64_t idx = (int64_t)blockIdx.x * kRowsWaves + wv; idx < a.ntasks;) {
+    lds_order();
+    const int start = a.row_ptr[idx], n = a.row_ptr[idx + 1] - start;
+    if (n <= kLongRow) run_task<NB, false, false>(a, Task{(int32_t)idx, start, n, -1}, lds, lane);
+    if (waves >= a.ntasks) break;  // (every row had its wavefront)
+    int more = 0;
+    if (lane == 0) more = atomicAdd(a.task_counter, 1);
+    idx = waves + __builtin_amdgcn_readfirstlane(more);
+  }
+}
+#endif
+
 constexpr int kFallbackGrid = 2048;  // work-groups walking the fallback list
 
 template <int NB>
@@ -253,6 +333,19 @@ static hipError_t launch_nb(const SweepArgs& a, hipStream_t s, int which) {
     if (a.nheavy > 0)
       hipLaunchKernelGGL((als_finish_kernel<NB, CG>), dim3((unsigned)a.nheavy), dim3(64), shmem, s, a);
   } else if constexpr (!CG) {
+#if CUMF_SWEEP_SOLVER == 0
+    if (which == 5) {
+      // whole rows without a plan (FP32), on at most a.persistent groups; a
+      // wavefront per row where there are fewer, and batches small enough that
+      // every group gets one or two of them
+      if (bf || a.persistent < 1 || a.ntasks < 1) return hipErrorInvalidValue;
+      const int64_t need = (a.ntasks + kRowsWaves - 1) / kRowsWaves;
+      const int64_t groups = need < a.persistent ? need : a.persistent;
+      const int64_t per = (a.ntasks + 2 * groups - 1) / (2 * groups);
+      const int batch = (int)(per > 64 ? 64 : per);
+      hipLaunchKernelGGL((als_rows_kernel<NB>), dim3((unsigned)groups), dim3(64 * kRowsWaves), 0, s, a, batch);
+    } else
+#endif
     if (which == 3) {
       // the CG path's Cholesky fallback (lives with the Cholesky kernels)
       const size_t shc = sizeof(float) * (size_t)lds_floats_nb(NB, bf);
@@ -310,6 +403,7 @@ hipError_t launch_finish_kernel(const SweepArgs& a, hipStream_t s) { return disp
 #if CUMF_SWEEP_SOLVER == 0
 hipError_t launch_fallback_kernel(const SweepArgs& a, hipStream_t s) { return dispatch(a, s, 3); }
 hipError_t launch_dual_kernel(const SweepArgs& a, hipStream_t s) { return dispatch(a, s, 4); }
+hipError_t launch_rows_kernel(const SweepArgs& a, hipStream_t s) { return dispatch(a, s, 5); }
 #endif
 
 }  // namespace CUMF_SNS

@@ -5,10 +5,11 @@
 // allocate or synchronise (code under HIP graph capture, tight serving
 // loops) use cumf_half_sweep_device_noalloc instead: same arithmetic (FP32
 // Gram on MFMA, FP32 Cholesky), no host work beyond argument checks, no
-// device allocation and no synchronisation.  A persistent grid of
-// wavefronts takes whole rows from a counter; the counter and the
-// failed-row count live in `scratch`, a file-scope device array of
-// kScratchInts ints that each GPU holds for the life of the process.
+// device allocation and no synchronisation.  One work-group per CU takes
+// whole rows from counters (long rows together, the others wavefront by
+// wavefront); the counters and the failed-row count live in `scratch`, a
+// file-scope device array of kScratchInts ints that each GPU holds for the
+// life of the process.
 //
 // The array's name is a host-side stand-in: its device address comes from
 // hipGetSymbolAddress, once per device, on the first call made with that
@@ -30,13 +31,14 @@ namespace {
 constexpr int kScratchInts = 64;  // see scratch below
 }  // namespace
 
-// [0] next row, [1] rows with a non-positive pivot; 256 bytes per GPU.
+// [0] next row, [1] rows with a non-positive pivot, [2] next batch of rows to
+// look for long ones in; 256 bytes per GPU.
 static __device__ __align__(256) int scratch[kScratchInts];
 
 namespace {
 constexpr int kMaxDevices = 64;
 constexpr int kMaxFusedF = 140;
-constexpr int64_t kMaxRows = INT_MAX - (1 << 20);  // the row counter may overshoot by one per wavefront
+constexpr int64_t kMaxRows = INT_MAX - (1 << 20);  // the counters may overshoot by one per wavefront
 
 __global__ void clear_scratch_kernel(int* p) {
   if (threadIdx.x < kScratchInts) p[threadIdx.x] = 0;
@@ -112,16 +114,16 @@ extern "C" int cumf_half_sweep_device_noalloc(hipStream_t stream, const int32_t*
   a.theta = d_theta;
   a.x = d_x;
   a.ldf = f;
-  a.tasks = nullptr;  // whole rows, taken in index order from the counter
+  a.tasks = nullptr;  // whole rows, taken in index order from the counters
   a.ntasks = m;
   a.fail_counter = ds.ptr + 1;
   a.f = f;
   a.lambda = lambda;
-  a.persistent = ds.num_cus * 4 * variant;  // one wavefront per SIMD per register-budget slot
+  a.persistent = ds.num_cus;  // at most one work-group per CU
   a.task_counter = ds.ptr;
   hipLaunchKernelGGL(clear_scratch_kernel, dim3(1), dim3(kScratchInts), 0, stream, ds.ptr);
   CUMF_HIP_TRY(hipGetLastError());
-  CUMF_HIP_TRY(variant == 1 ? cumf::w1::chol::launch_task_kernel(a, stream)
-                            : cumf::w2::chol::launch_task_kernel(a, stream));
+  CUMF_HIP_TRY(variant == 1 ? cumf::w1::chol::launch_rows_kernel(a, stream)
+                            : cumf::w2::chol::launch_rows_kernel(a, stream));
   return CUMF_OK;
 }

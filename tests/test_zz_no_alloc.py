@@ -66,3 +66,35 @@ def test_noalloc_rejects_unsupported_shapes():
         rc = L.cumf_half_sweep_device_noalloc(None, rp.ctypes.data, rp.ctypes.data, rp.ctypes.data, rp.ctypes.data,
                                               rp.ctypes.data, 1, 1, f, 1, 0.1)
         assert rc == 1 and "multiple of 4" in G.last_error()
+
+
+# One to nine column blocks; f = 128 and 140 run four wavefronts a group, the
+# others eight.
+@pytest.mark.parametrize("f", [4, 16, 44, 64, 100, 108, 128, 140])
+@pytest.mark.parametrize("m", [1, 37, 700])
+def test_noalloc_long_rows(f, m):
+    """Rows of more than 2,048 ratings, solved by a work-group together: lengths
+    at the edge, with empty and uneven shares, several in one batch of rows.
+    Each row's relative residual against the FP64 system on its factors is at
+    most 1e-5; the shorter rows equal the allocating path's bit for bit."""
+    n, lam = 12000, 0.05
+    rng = np.random.default_rng(f * 1000 + m)
+    counts = rng.integers(0, 60, m)
+    longs = np.array([2048, 2049, 2080, 2081, 2303, 4096, 7001, 11999])
+    counts[rng.choice(m, min(m, 8), replace=False)] = longs[:min(m, 8)] if m > 1 else 2049
+    if m > 20:
+        counts[3:6] = [3000, 2500, 2049]
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ci = np.concatenate([rng.choice(n, c, replace=False) for c in counts]).astype(np.int32)
+    cv = rng.integers(1, 6, rp[-1]).astype(np.float32)
+    theta = cumf.init_factors(n, f, 3)
+    Xn = _sweep(True, rp, ci, cv, theta, f, lam)
+    Xa = _sweep(False, rp, ci, cv, theta, f, lam)
+    whole = counts <= 2048
+    np.testing.assert_array_equal(Xn[whole], Xa[whole])
+    for u in np.flatnonzero(~whole):
+        Y = theta[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+        b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+        x = Xn[u].astype(np.float64)
+        res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(counts[u])) * x
+        assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, u, counts[u])
