@@ -84,11 +84,7 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
   gram_any<NB, BF>(acc, a, (int64_t)t.start, t.count, lds, lane);
 
   if (t.slot >= 0) {  // partial Gram of a heavy row
-    float* dst = a.partial + (int64_t)t.slot * num_tiles(NB) * 256;
-#pragma unroll
-    for (int i = 0; i < num_tiles(NB); ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dst[(i * 4 + r) * 64 + lane] = acc[i][r];
+    store_partial<NB>(a.partial + (int64_t)t.slot * num_tiles(NB) * 256, acc, lane);
     return;
   }
   add_ridge<NB>(acc, a.f, a.lambda * (float)t.count, lane);
@@ -125,15 +121,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
   const HeavyRow h = a.heavy[blockIdx.x];
   if (h.row < 0) return;
   f4 acc[num_tiles(NB)];
-#pragma unroll
-  for (int i = 0; i < num_tiles(NB); ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < h.nchunks; ++p) {
-    const float* src = a.partial + (int64_t)(h.slot + p) * num_tiles(NB) * 256;
-#pragma unroll
-    for (int i = 0; i < num_tiles(NB); ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][r] += src[(i * 4 + r) * 64 + lane];
-  }
+  sum_partials<NB>(acc, a.partial, h, lane);
   const int n_u = a.row_ptr[h.row + 1] - a.row_ptr[h.row];
   add_ridge<NB>(acc, a.f, a.lambda * (float)n_u, lane);
   const bool bf = a.precision != 0;
@@ -172,13 +160,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
     } else {
       const HeavyRow h = a.heavy[-1 - e];
       row = h.row;
-      for (int p = 0; p < h.nchunks; ++p) {
-        const float* src = a.partial + (int64_t)(h.slot + p) * num_tiles(NB) * 256;
-#pragma unroll
-        for (int i = 0; i < num_tiles(NB); ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][r] += src[(i * 4 + r) * 64 + lane];
-      }
+      sum_partials<NB>(acc, a.partial, h, lane);
     }
     const int n_u = a.row_ptr[row + 1] - a.row_ptr[row];
     add_ridge<NB>(acc, a.f, a.lambda * (float)n_u, lane);
@@ -202,11 +184,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
   if (t.slot >= 0) {
     f4 acc[num_tiles(NB)];
     gram_any<NB, true>(acc, a, (int64_t)t.start, t.count, lds, lane);
-    float* dst = a.partial + (int64_t)t.slot * num_tiles(NB) * 256;
-#pragma unroll
-    for (int i = 0; i < num_tiles(NB); ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dst[(i * 4 + r) * 64 + lane] = acc[i][r];
+    store_partial<NB>(a.partial + (int64_t)t.slot * num_tiles(NB) * 256, acc, lane);
     return;
   }
   dual_solve_row<NB, CH>(a, t, lds, lane);
