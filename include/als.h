@@ -107,8 +107,9 @@ typedef struct cumf_options {
   int32_t precision;    /* CUMF_PREC_* */
   int32_t split;        /* max ratings per wavefront task; longer rows are
                            split and their partial Grams reduced (0: 16384).
-                           The device entry points cut finer where a matrix
-                           is too small to fill the GPU with such tasks */
+                           Without a tile table rows are cut finer (not
+                           below 2048) where a matrix is too small to fill
+                           the GPU with such tasks */
   int32_t timing;       /* 1: time every kernel launch with HIP events */
   int32_t use_graph;    /* 1: each half-sweep (X, Theta) is replayed from a
                            hipGraph captured at its first run; per-kernel
