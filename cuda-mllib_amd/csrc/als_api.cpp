@@ -7,7 +7,8 @@
 // wavefront tasks, then the reduction of split rows), with the ratings and
 // both factor matrices resident on the device between sweeps.
 //
-// Task planning (host, once per rating matrix): every row with at most
+// Task planning (for a resident handle on the host, once per rating matrix;
+// for the device entry points on the device, planner.hip): every row with at most
 // `split` ratings becomes one task; longer rows are cut into `split`-sized
 // chunks whose partial Grams land in scratch slots and are summed in chunk
 // order by the finish kernel.  Tasks are ordered by decreasing length so
@@ -204,9 +205,8 @@ struct DevicePlan {
 // Longest task of a matrix of nnz ratings: the caller's split size, less
 // where that would leave the chip waiting for one wavefront.  A task is at
 // most half of a wavefront's share when 2,048 of them (two per SIMD) run side
-// by side, and never under 2,048 ratings (a row of 2,048 costs a wavefront
-// about 0.1 ms at f = 100; finer cuts cost more in partial Grams than they
-// save).  Measured at 60,023 x 17,770, 12.4 million ratings, f = 50: the task
+// by side, and never under 2,048 ratings (the entry point that cannot split
+// solves rows up to that length whole, with the same result).  Measured at 60,023 x 17,770, 12.4 million ratings, f = 50: the task
 // kernel 1.45 ms with a 16,384-rating task at its head; the whole call 0.85 ms
 // with 3,023.
 int adaptive_split(int split, int64_t nnz) {

@@ -5,7 +5,7 @@
 // The device entry points get a rating matrix per call, so its plan is part
 // of every call.  Read back and sorted on the host, the plan of 480,189 rows
 // took 18 ms beside a half-sweep of 16.5 ms; here it is a counting sort in
-// device memory, 0.03 ms, and nothing but the summary crosses the bus.
+// device memory, 0.04 ms, and nothing but the summary crosses the bus.
 //
 // Same tasks as plan_tasks: a row of at most `split` ratings is one task, a
 // longer one ceil(n / split) chunks of near-equal size in consecutive

@@ -71,7 +71,7 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
 
 #define CUMF_OPTIONS_VERSION 1
 
-#define CUMF_PREC_FP32 0        /* FP32 Gram on MFMA, FP32 Cholesky */
+#define CUMF_PREC_FP32 0        /* FP32 Gram (split BF16 products), FP32 Cholesky */
 #define CUMF_PREC_BF16_GRAM 1   /* Gram on BF16 MFMA (FP32 accumulation) from BF16
                                    copies of the factors, b from a BF16 hi/lo split
                                    of the ratings, FP32 Cholesky */
