@@ -2047,8 +2047,8 @@ __device__ __forceinline__ void fp32_dual_row(const SweepArgs& a, const Task& t,
 }
 
 // Row blocks of the dual system up to which the FP32 task kernel takes it in
-// place of the f x f system of NB blocks (0: never; 6: 95 ratings): wherever it
-// is the smaller one.  Measured, 480,189 x 17,770, f = 100, where 315,077 rows
+// place of the f x f system of NB blocks (0: never; 6: 95 ratings), given a
+// ridge: wherever it is the smaller one.  Measured, 480,189 x 17,770, f = 100, where 315,077 rows
 // have at most 95 ratings: X half-sweep 12.0 -> 10.1 ms; 60,023 x 17,770,
 // f = 128 3.4 -> 2.8 ms, f = 50 0.66 -> 0.65 ms.  A line one block lower gave
 // the same within 1%, two blocks lower 10.5 ms at f = 100 and 0.25 against

@@ -526,3 +526,23 @@ def test_short_rows_on_both_sides_of_the_dual_line(f):
         x = X[u].astype(np.float64)
         res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(counts[u])) * x
         assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, u, np.linalg.norm(res) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("f", [20, 100, 140])
+def test_singular_rows_without_a_ridge_fail_as_before(f):
+    """lambda = 0 and fewer ratings than f: the f x f system is singular.  Rows
+    of unit-vector factors have an exactly zero pivot: x = 0, counted, though
+    their n x n system could be solved."""
+    n = f
+    T = np.eye(n, f, dtype=np.float32)
+    rp = np.array([0, 1, 4, 4 + f], np.int32)
+    ci = np.concatenate([[3], [1, 2, 5], np.arange(f)]).astype(np.int32)
+    cv = np.full(4 + f, 2.0, np.float32)
+    with G.ALS(f, 0.0) as h:
+        h.set_ratings(3, n, rp, ci, cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 2
+    assert np.all(X[:2] == 0)
+    np.testing.assert_allclose(X[2], 2.0, rtol=1e-6)
