@@ -1922,6 +1922,21 @@ struct CacheLease {
   }
 };
 
+// Waits for a stream when the scope ends, unless done() was called: a call
+// that fails half way gives its device's cache back only once nothing of it
+// is under way.
+struct SyncOnFailure {
+  hipStream_t s;
+  bool armed = true;
+  explicit SyncOnFailure(hipStream_t stream) : s(stream) {}
+  SyncOnFailure(const SyncOnFailure&) = delete;
+  SyncOnFailure& operator=(const SyncOnFailure&) = delete;
+  ~SyncOnFailure() {
+    if (armed) (void)hipStreamSynchronize(s);
+  }
+  void done() { armed = false; }
+};
+
 // Where the bound on a matrix's partial Grams is at most this, they are sized
 // by the bound and the sweep is launched behind the planner without waiting
 // for it; above it the host waits for the plan's counts (about 15 us).
@@ -1978,6 +1993,7 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
     cumf::set_last_error("hipHostMalloc of the plan summary failed");
     return CUMF_ERR_NOMEM;
   }
+  SyncOnFailure pending(stream);
   CUMF_HIP_TRY(cumf::launch_plan(d_row_ptr, m, nnz, split, plan.tasks.as<cumf::Task>(), task_cap,
                                  plan.heavy.as<cumf::HeavyRow>(), heavy_cap, plan.work.p, plan.summary, stream));
   // Refuses row pointers that do not start at 0, end at nnz and never
@@ -2054,8 +2070,9 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
   }
   if (ldf != f)
     CUMF_HIP_TRY(cumf::launch_restride(x, ldf, d_x, f, m, f, stream));
-  if (!wait) return check_plan();
-  CUMF_HIP_TRY(hipStreamSynchronize(stream));
+  if (!wait) CUMF_TRY(check_plan());
+  else CUMF_HIP_TRY(hipStreamSynchronize(stream));
+  pending.done();
   return CUMF_OK;
 }
 
@@ -2092,6 +2109,7 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
     const size_t tb = sizeof(float) * (size_t)n * f, xb = sizeof(float) * (size_t)m * f;
     CUMF_TRY(ensure(theta, tb));
     CUMF_TRY(ensure(x, xb));
+    SyncOnFailure pending(cuda_stream);
     CUMF_HIP_TRY(hipMemcpyAsync(theta.p, thetaTHost, tb, hipMemcpyHostToDevice, cuda_stream));
     cumf_options o;
     cumf_default_options(&o);
@@ -2101,6 +2119,7 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
                                m, n, f, nnz, lambda, &o, lease.c));
     CUMF_HIP_TRY(hipMemcpyAsync(XTHost, x.p, xb, hipMemcpyDeviceToHost, cuda_stream));
     CUMF_HIP_TRY(hipStreamSynchronize(cuda_stream));
+    pending.done();
     return CUMF_OK;
   };
   int rc = run();
