@@ -2055,4 +2055,18 @@ __device__ __forceinline__ void fp32_dual_row(const SweepArgs& a, const Task& t,
 // 0.22 ms at f = 32 (50 ratings a row).
 __host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB - 1 > 6 ? 6 : NB - 1; }
 
+// Whether the kernels of NB blocks solve a whole FP32 row of n ratings in the
+// dual form.  Besides the line above:
+//   * a ridge: without one the f x f system of so short a row is singular and
+//     the row fails; its n x n one need not be;
+//   * n <= f (in the last block column f may be up to 3 below n): Y Y^T has
+//     rank f, so with more ratings than that only the ridge keeps it from
+//     being singular, where Y^T Y needs none.  Errors against 64 bits at
+//     f = 13, 14 ratings a row: 2e-4 against 4e-5 at lambda = 1e-5, 2e-2
+//     against 6e-5 at 1e-7, and failed rows below that.
+template <int NB>
+__device__ __forceinline__ bool fp32_takes_dual(const SweepArgs& a, int n) {
+  return a.lambda > 0.0f && n <= 16 * fp32_dual_max_blocks(NB) - 1 && n <= a.f;
+}
+
 }  // namespace cumf

@@ -65,9 +65,7 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
   }
 
   if constexpr (!BF && !CG && fp32_dual_max_blocks(NB) > 0) {
-    // (Without a ridge the f x f system of so short a row is singular and the
-    // row fails; its n x n one need not be.)
-    if (t.slot < 0 && a.lambda > 0.0f && t.count <= 16 * fp32_dual_max_blocks(NB) - 1) {
+    if (t.slot < 0 && fp32_takes_dual<NB>(a, t.count)) {
       fp32_dual_row<fp32_dual_max_blocks(NB)>(a, t, lds, lane);
       return;
     }
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
       const int cnt = a.row_ptr[row + 1] - a.row_ptr[row];
       lds_order();
       if constexpr (!BF && fp32_dual_max_blocks(NB) > 0) {  // as the task kernel solves them
-        if (cnt > 0 && a.lambda > 0.0f && cnt <= 16 * fp32_dual_max_blocks(NB) - 1) {
+        if (cnt > 0 && fp32_takes_dual<NB>(a, cnt)) {
           fp32_dual_row<fp32_dual_max_blocks(NB)>(a, Task{(int32_t)row, (int32_t)s, cnt, -1}, lds, lane);
           continue;
         }

@@ -546,3 +546,30 @@ def test_singular_rows_without_a_ridge_fail_as_before(f):
         assert h.stats()["failed_rows"] == 2
     assert np.all(X[:2] == 0)
     np.testing.assert_allclose(X[2], 2.0, rtol=1e-6)
+
+
+@pytest.mark.parametrize("f", [13, 14, 29, 45, 61, 77, 93, 94])
+def test_rows_of_more_ratings_than_rank_keep_their_system(f):
+    """A few more ratings than f, orthonormal factor columns and next to no
+    ridge: Y^T Y is the identity (any FP32 solve of it is good to 1e-5, the
+    plain path's bar), Y Y^T has rank f < n and is singular but for 1e-6 of a
+    ridge."""
+    lam = 1e-7
+    rng = np.random.default_rng(f)
+    counts = list(range(f + 1, f + 8))  # the dual form ends at a block edge up to 3 past f
+    n, m = sum(counts), len(counts)
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    T = np.concatenate([np.linalg.qr(rng.standard_normal((c, f)))[0] for c in counts]).astype(np.float32)
+    cv = rng.integers(1, 6, n).astype(np.float32)
+    with G.ALS(f, lam) as h:
+        h.set_ratings(m, n, rp, np.arange(n, dtype=np.int32), cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 0
+    for u, cnt in enumerate(counts):
+        Y = T[rp[u]:rp[u + 1]].astype(np.float64)
+        b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+        x = X[u].astype(np.float64)
+        res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(cnt)) * x
+        assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, cnt, np.linalg.norm(res) / np.linalg.norm(b))
