@@ -154,13 +154,20 @@ __device__ __forceinline__ void lds_order() {
 static __device__ const float kZeroRow[256] = {};
 
 // ---------------------------------------------------------------------------
-// FP32 products on the BF16 matrix pipe.  A float is the sum of three BF16
-// values h + m + l: h its upper half (truncated), m the remainder rounded to
-// BF16, l what is left, which is at most 8 bits and exact.  Of the nine
-// products of two such sums the six hh, hm, mh, mm, hl, lh carry the FP32
-// product to about 2^-24; ml, lm and ll are left out.  Six
-// v_mfma_f32_16x16x32_bf16 (16 cycles of the matrix pipe each) do 32 k-values
-// where eight v_mfma_f32_16x16x4_f32 take 32 cycles each.
+// FP32 products on the BF16 matrix pipe (the three-way split of Henry, Tang
+// and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", ARITH 2019).  A float is the sum of three
+// BF16 values h + m + l: h its upper half (truncated), m the remainder rounded
+// to BF16, l what is left, which is at most 8 bits and exact.  With 2^e the
+// leading power of two, |m| <= 2^(e-7) and |l| <= 2^(e-16).  Of the nine
+// products of two such sums the six hh, hm, mh, mm, hl, lh are taken; ml, lm
+// and ll are left out: at most 2^-22 of a product (about 2^-25.5 rms on random
+// operands; a product rounded to FP32 is off by at most 2^-24).  A sum gains
+// more than that from fewer roundings (split_tiles).  Rounding h instead would
+// leave out at most 2^-24, for 1 to 7% of every FP32 half-sweep, and moved no
+// error of a whole row above one block.  Six v_mfma_f32_16x16x32_bf16 (16
+// cycles of the matrix pipe each) do 32 k-values where eight
+// v_mfma_f32_16x16x4_f32 take 32 cycles each.
 // ---------------------------------------------------------------------------
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
@@ -2047,13 +2054,21 @@ __device__ __forceinline__ void fp32_dual_row(const SweepArgs& a, const Task& t,
 }
 
 // Row blocks of the dual system up to which the FP32 task kernel takes it in
-// place of the f x f system of NB blocks (0: never; 6: 95 ratings), given a
-// ridge: wherever it is the smaller one.  Measured, 480,189 x 17,770, f = 100, where 315,077 rows
+// place of the f x f system of NB blocks (6: 95 ratings), given a ridge:
+// wherever it is the smaller one.  Measured, 480,189 x 17,770, f = 100, where 315,077 rows
 // have at most 95 ratings: X half-sweep 12.0 -> 10.1 ms; 60,023 x 17,770,
 // f = 128 3.4 -> 2.8 ms, f = 50 0.66 -> 0.65 ms.  A line one block lower gave
 // the same within 1%, two blocks lower 10.5 ms at f = 100 and 0.25 against
 // 0.22 ms at f = 32 (50 ratings a row).
-__host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB - 1 > 6 ? 6 : NB - 1; }
+__host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB > 7 ? 6 : NB > 1 ? NB - 1 : 1; }
+// Longest row it takes.  One block (f <= 12) takes it for accuracy: the
+// entries of a Gram of one or two ratings are single products, whose split is
+// off by up to 2^-22.  Error against 64 bits at f = 4 / 12, rms: one rating
+// 7.1e-7 / 5.7e-7 in the f x f system (5.8e-7 / 5.0e-7 with plain FP32
+// products), 8.2e-8 / 8.3e-8 in this one; from four ratings on the f x f
+// system is ahead of plain FP32 products.  600,000 rows of one to four
+// ratings: 446 -> 419 .. 433 us at f = 12.
+__host__ __device__ constexpr int fp32_dual_max_ratings(int NB) { return NB > 1 ? 16 * fp32_dual_max_blocks(NB) - 1 : 4; }
 
 // Whether the kernels of NB blocks solve a whole FP32 row of n ratings in the
 // dual form.  Besides the line above:
@@ -2066,7 +2081,7 @@ __host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB - 1 >
 //     against 6e-5 at 1e-7, and failed rows below that.
 template <int NB>
 __device__ __forceinline__ bool fp32_takes_dual(const SweepArgs& a, int n) {
-  return a.lambda > 0.0f && n <= 16 * fp32_dual_max_blocks(NB) - 1 && n <= a.f;
+  return a.lambda > 0.0f && n <= fp32_dual_max_ratings(NB) && n <= a.f;
 }
 
 }  // namespace cumf

@@ -64,7 +64,7 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
     return;
   }
 
-  if constexpr (!BF && !CG && fp32_dual_max_blocks(NB) > 0) {
+  if constexpr (!BF && !CG) {
     if (t.slot < 0 && fp32_takes_dual<NB>(a, t.count)) {
       fp32_dual_row<fp32_dual_max_blocks(NB)>(a, t, lds, lane);
       return;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
       const int64_t s = a.row_ptr[row];
       const int cnt = a.row_ptr[row + 1] - a.row_ptr[row];
       lds_order();
-      if constexpr (!BF && fp32_dual_max_blocks(NB) > 0) {  // as the task kernel solves them
+      if constexpr (!BF) {  // as the task kernel solves them
         if (cnt > 0 && fp32_takes_dual<NB>(a, cnt)) {
           fp32_dual_row<fp32_dual_max_blocks(NB)>(a, Task{(int32_t)row, (int32_t)s, cnt, -1}, lds, lane);
           continue;

@@ -573,3 +573,26 @@ def test_rows_of_more_ratings_than_rank_keep_their_system(f):
         x = X[u].astype(np.float64)
         res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(cnt)) * x
         assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, cnt, np.linalg.norm(res) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("f", [1, 2, 3, 4, 7, 8, 10, 12])
+def test_rows_of_one_rating_at_small_ranks(f):
+    """One rating r with factor y: x = r y / (|y|^2 + lambda).  Solved as that
+    1 x 1 system it is off by at most 16 * 2^-24: 4 for the products left out
+    of the split of |y|^2, 4 for the rounding of its matrix instructions (two
+    of full size, one ulp each), 6 for the pivot's reciprocal square root taken
+    twice, 2 for the ridge and the last product."""
+    m, n, lam = 4000, 2000, 0.05
+    rng = np.random.default_rng(f)
+    T = (0.3 + rng.standard_normal((n, f))).astype(np.float32) / np.float32(np.sqrt(f))
+    ci = rng.integers(0, n, m).astype(np.int32)
+    cv = rng.integers(1, 6, m).astype(np.float32)
+    with G.ALS(f, lam) as h:
+        h.set_ratings(m, n, np.arange(m + 1, dtype=np.int32), ci, cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+    Y = T[ci].astype(np.float64)
+    want = cv[:, None] * Y / ((Y * Y).sum(1, keepdims=True) + float(np.float32(lam)))
+    err = np.linalg.norm(X - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert err.max() <= 16 * 2.0 ** -24, err.max()
