@@ -60,8 +60,9 @@ std::atomic<int> g_large_dual{1};
 // Launch shape of one bucket: register budget (wavefronts per SIMD the
 // kernel was compiled for, 1 or 2), persistent grid (0: one work-group per
 // task; > 0: that many wavefronts taking tasks from a counter) and solver
-// (-1: the handle's; CUMF_SOLVER_CHOLESKY or CUMF_SOLVER_CG, which the
-// autotuner may pick per bucket when the handle's solver is CG).
+// (-1: the handle's; CUMF_SOLVER_CHOLESKY, on FP32 factors the f x f system
+// of every row where -1 takes short rows in the dual form; CUMF_SOLVER_CG,
+// which the autotuner may pick per bucket when the handle's solver is CG).
 struct BucketCfg {
   int variant = 2;
   int persistent = 0;
@@ -414,6 +415,11 @@ static_assert(kBucketEdge[kDualBuckets] == cumf::kDualMaxRatingsHost + 1, "dual-
 // two up to 63, three up to 95.
 int dual_chunks_of(int b) { return kBucketEdge[b + 1] <= 32 ? 1 : kBucketEdge[b + 1] <= 64 ? 2 : 3; }
 
+// Whether a bucket's launch keeps the f x f system of short FP32 rows.
+int primal_of(const cumf::SweepArgs& a, const BucketCfg& cfg) {
+  return a.precision == CUMF_PREC_FP32 && cfg.solver == CUMF_SOLVER_CHOLESKY;
+}
+
 // Launch of the tasks of degree buckets b_lo .. b (a contiguous range of the
 // task list: tasks are ordered by decreasing rating count) with one shape.
 hipError_t bucket_launch(cumf_handle* h, int side, const Plan& p, const cumf::SweepArgs& a, int b,
@@ -445,6 +451,7 @@ hipError_t bucket_launch(cumf_handle* h, int side, const Plan& p, const cumf::Sw
     return dual_launch(x, cfg.variant, stream);
   }
   if (cfg.solver >= 0) x.solver = cfg.solver;
+  x.primal = primal_of(x, cfg);
   return task_launch(x, cfg.variant, stream);
 }
 
@@ -512,7 +519,7 @@ int launch_tasks(cumf_handle* h, int side, const Plan& p, const cumf::SweepArgs&
   if (!h->tiled) return timed(h, Timer::TASK, [&] { return task_launch(a, default_variant(h->f), h->stream); });
   // A side whose non-empty buckets share one shape and no persistent grid is
   // one launch (launches in sequence drain the GPU between buckets).
-  int v0 = 0, s0 = -2, o0 = 0;
+  int v0 = 0, s0 = -2, o0 = 0, p0 = 0;
   bool uniform = true;
   for (int b = 0; b < kBuckets; ++b) {
     if (p.bucket_t1[b] <= p.bucket_t0[b]) continue;
@@ -522,13 +529,15 @@ int launch_tasks(cumf_handle* h, int side, const Plan& p, const cumf::SweepArgs&
       v0 = c.variant;
       s0 = sv;
       o0 = c.occupancy;
+      p0 = primal_of(a, c);
     }
-    uniform = uniform && c.persistent == 0 && c.variant == v0 && sv == s0 && c.occupancy == o0;
+    uniform = uniform && c.persistent == 0 && c.variant == v0 && sv == s0 && c.occupancy == o0 && primal_of(a, c) == p0;
   }
   if (uniform && v0 != 0 && s0 != CUMF_SOLVER_DUAL) {
     cumf::SweepArgs x = a;
     x.solver = s0;
     x.occupancy = o0;
+    x.primal = p0;
     return timed(h, Timer::TASK, [&] { return task_launch(x, v0, h->stream); });
   }
   bool persistent = false;
@@ -1411,7 +1420,11 @@ int autotune_side(cumf_handle* h, int side, int reps, const TuneStart& start) {
     double bk = 1e300;
     BucketCfg bc;
     std::vector<int> sols = solvers;
-    if (k < kDualBuckets) sols.push_back(CUMF_SOLVER_DUAL);
+    if (k < kDualBuckets) {
+      // (on FP32 factors -1 already takes rows in the dual form by length)
+      if (!cg && h->opt.precision == CUMF_PREC_FP32) sols.push_back(CUMF_SOLVER_CHOLESKY);
+      sols.push_back(CUMF_SOLVER_DUAL);
+    }
     for (int sol : sols)
       for (int variant : {2, 1})
         for (int pers : {0, h->num_cus * (variant == 1 ? 4 : 8), -7, -6, -3}) {

@@ -2071,7 +2071,8 @@ __host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB > 7 ?
 __host__ __device__ constexpr int fp32_dual_max_ratings(int NB) { return NB > 1 ? 16 * fp32_dual_max_blocks(NB) - 1 : 4; }
 
 // Whether the kernels of NB blocks solve a whole FP32 row of n ratings in the
-// dual form.  Besides the line above:
+// dual form.  Besides the line above, and unless the launch is a tile table's
+// Cholesky one:
 //   * a ridge: without one the f x f system of so short a row is singular and
 //     the row fails; its n x n one need not be;
 //   * n <= f (in the last block column f may be up to 3 below n): Y Y^T has
@@ -2081,7 +2082,7 @@ __host__ __device__ constexpr int fp32_dual_max_ratings(int NB) { return NB > 1 
 //     against 6e-5 at 1e-7, and failed rows below that.
 template <int NB>
 __device__ __forceinline__ bool fp32_takes_dual(const SweepArgs& a, int n) {
-  return a.lambda > 0.0f && n <= fp32_dual_max_ratings(NB) && n <= a.f;
+  return !a.primal && a.lambda > 0.0f && n <= fp32_dual_max_ratings(NB) && n <= a.f;
 }
 
 }  // namespace cumf

@@ -65,6 +65,9 @@ struct SweepArgs {
   // -1 - index into heavy for a split row; fb_count = list length.
   int* fb_list;
   int* fb_count;
+  // != 0: FP32 rows in the f x f system whatever their length (a tile table's
+  // Cholesky); 0: short ones in the dual form.
+  int primal;
   // persistent > 0: launch that many wavefronts, each taking tasks from
   // *task_counter (zero before the launch) until ntasks are taken.
   // launch_rows_kernel: that many work-groups over the rows 0 .. ntasks of

@@ -89,8 +89,8 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
                                    most 95 ratings): the same x from the n x n
                                    system (Y Y^T + lambda n I) z = r, x = Y^T z,
                                    with Y the row's n gathered factor rows (K
-                                   on BF16 MFMA from the BF16 copies, or on FP32
-                                   MFMA from the factors on a CUMF_PREC_FP32
+                                   on BF16 MFMA from the BF16 copies, or in split
+                                   BF16 products from the factors on a CUMF_PREC_FP32
                                    handle; FP32 Cholesky of the smaller system).
                                    On an FP32 handle a launch holding a split
                                    row's chunk takes the Cholesky kernel */
@@ -145,7 +145,10 @@ typedef struct cumf_stats {
   int64_t rmse_launches;
   double sweep_ms;         /* whole half-sweeps, first to last kernel */
   int64_t sweeps;
-  int64_t failed_rows;     /* rows with a non-positive pivot (x_u set to 0) */
+  int64_t failed_rows;     /* rows with a non-positive pivot (x_u set to 0): with fewer
+                              ratings than f and lambda too small for FP32, rows
+                              solved in the f x f system fail where the dual form
+                              still solves them */
   int64_t gram_flops;      /* nnz f(f+1) (the f(f+1)/2 unique Gram entries, one
                               multiply-add each, per rating) summed over the
                               half-sweeps run */
@@ -264,7 +267,9 @@ int cumf_csr_to_csc_device(hipStream_t stream, int64_t m, int64_t n, int64_t nnz
  * fallback kernels, and per bucket the register budget, whether the bucket
  * runs as a persistent grid of N wavefronts taking tasks from a counter, its
  * solver (the handle's, Cholesky, the dual form in buckets 0-2, or -- on a
- * CG handle -- CG), and a cap on
+ * CG handle -- CG; on a CUMF_PREC_FP32 handle the handle's Cholesky takes
+ * rows of few ratings in the dual form by itself, and Cholesky by name the
+ * f x f system of every row), and a cap on
  * the wavefronts per CU of a one-task-per-group launch (3..16; 0 = none),
  * enforced through the LDS each group requests.  Without
  * a table every half-sweep is one launch of all tasks,

@@ -306,3 +306,45 @@ def test_batched_graph_half_sweeps_match_oracle(tmp_path, solver, precision):
     # the factor error is the residual times the system's conditioning
     ebar = 1e-3 if solver == G.CUMF_SOLVER_CHOLESKY else 1e-2
     assert ex.max() <= ebar and et.max() <= ebar, (ex.max(), et.max())
+
+
+@pytest.mark.parametrize("f", [10, 32, 100])
+def test_fp32_table_cholesky_is_the_primal_system(tmp_path, f):
+    """On an FP32 handle a table's solver 0 solves short rows in the f x f
+    system, 2 and -1 in the n x n one.  With an ordinary ridge all agree to
+    1e-4; next to none (1e-12, far below FP32's rounding of the f x f
+    system's zero pivots) the f x f system of a row of fewer ratings than f
+    fails, x = 0 and counted, and the n x n one is solved to a residual of
+    1e-5 (its rows are orthonormal)."""
+    m, n, k = 40, 400, min(f - 1, 4 if f <= 12 else 20)
+    rng = np.random.default_rng(f)
+    rp = np.arange(0, k * m + 1, k, dtype=np.int32)
+    ci = np.concatenate([rng.choice(n // k, 1) * k + np.arange(k) for _ in range(m)]).astype(np.int32)
+    cv = rng.integers(1, 6, k * m).astype(np.float32)
+    T = np.concatenate([np.linalg.qr(rng.standard_normal((f, k)))[0].T for _ in range(n // k)]).astype(np.float32)
+
+    def solve(lam, solver):
+        tab = tmp_path / f"t{solver}.txt"
+        tab.write_text("".join(f"side {s} split 16384 finish 2 fallback 2\n" +
+                               "".join(f"bucket {s} {b} 0 0 variant 2 persistent 0 solver {solver if b < 3 else -1}\n"
+                                       for b in range(8)) for s in (0, 1)))
+        with G.ALS(f, lam) as h:
+            h.set_ratings(m, n, rp, ci, cv)
+            h.load_tile_table(str(tab))
+            h.set_factors(theta=T)
+            h.update_x()
+            return h.get_factors()[0], h.stats()["failed_rows"]
+
+    X = {s: solve(0.05, s) for s in (-1, 0, 2)}
+    assert all(bad == 0 for _, bad in X.values())
+    assert _rel(X[0][0], X[2][0]) <= 1e-4 and _rel(X[-1][0], X[2][0]) <= 1e-4
+    X0, bad = solve(1e-12, 0)
+    assert bad == m and np.all(X0 == 0)
+    for s in (-1, 2):
+        X1, bad = solve(1e-12, s)
+        assert bad == 0
+        for u in range(m):
+            Y = T[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+            b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+            res = b - Y.T @ (Y @ X1[u].astype(np.float64))
+            assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (s, u)
