@@ -295,13 +295,13 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
   static_assert(NBUF % 2 == 0, "chunks are taken in pairs");
   const bool last_in = 16 * (NB - 1) + 4 * sq < (int)ldf;
   const bool rating_lane = 16 * (NB - 1) + c == (int)ldf;
-  const int nch = (count + KB - 1) / KB;
+  const int nch = chunks_of(count, KB);
 
   // Column index of this lane's staging row in chunk ch (-1 past the end).
   auto load_ci = [&](int ch) -> int {
-    const int k = ch * KB + sr;
-    const int ci = col[start + (k < count ? k : count - 1)];
-    return k < count ? ci : -1;
+    const uint32_t k = position_in(ch, KB, sr), n = count;
+    const int ci = col[start + (k < n ? k : n - 1)];
+    return k < n ? ci : -1;
   };
   auto issue = [&](int ch, int buf, int ci) {
     float* yb = lds + buf * CF;
@@ -311,8 +311,8 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
       __builtin_amdgcn_global_load_lds(rp + 16 * I, (lds_void_t*)(yb + I * 256), 16, 0, 0);
     const float* rl = (last_in && ci >= 0) ? rp + 16 * (NB - 1) : kZeroRow;
     __builtin_amdgcn_global_load_lds(rl, (lds_void_t*)(yb + (NB - 1) * 256), 16, 0, 0);
-    const int k = ch * KB + lane;
-    const float* vp = (lane < KB && k < count) ? val + start + k : kZeroRow;
+    const uint32_t k = position_in(ch, KB, lane);
+    const float* vp = (lane < KB && k < (uint32_t)count) ? val + start + k : kZeroRow;
     __builtin_amdgcn_global_load_lds(vp, (lds_void_t*)(yb + NB * 256), 4, 0, 0);
   };
 

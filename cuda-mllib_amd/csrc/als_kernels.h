@@ -85,6 +85,13 @@ struct SweepArgs {
   int dual_partial;
 };
 
+// A range of count >= 1 ratings in chunks of `size`: how many there are, and
+// the position of a chunk's i-th rating, to be compared with the count as an
+// unsigned number.  Exact up to INT_MAX ratings and for the few chunks past
+// the end that a prefetch asks about, whose positions no longer fit an int.
+__host__ __device__ constexpr int chunks_of(int count, int size) { return (count - 1) / size + 1; }
+__host__ __device__ constexpr uint32_t position_in(int ch, int size, int i) { return (uint32_t)ch * size + i; }
+
 // Longest row the dual form takes (three staged chunks of 32 ratings).
 constexpr int kDualMaxRatingsHost = 95;
 

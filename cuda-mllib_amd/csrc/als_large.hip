@@ -137,16 +137,16 @@ __device__ __forceinline__ void gram_tiles(const SweepArgs& a, int64_t start, in
   const int ldf = (int)a.ldf;
   const bool last_in = 16 * (NB - 1) + 4 * sq < ldf;
   const int rcol = ldf - 16 * (NB - 1);  // the rating's column in the last tile
-  const int nst = (count + 2 * KB - 1) / (2 * KB);
+  const int nst = chunks_of(count, 2 * KB);
   f4 acc[Q];
 
   auto load_ci = [&](int st, int h) -> int {
-    const int k = 2 * KB * st + KB * h + sr;
-    return k < count ? a.col[start + k] : -1;
+    const uint32_t k = position_in(st, 2 * KB, KB * h + sr);
+    return k < (uint32_t)count ? a.col[start + k] : -1;
   };
   auto load_r = [&](int st) -> float {
-    const int k = 2 * KB * st + lane;
-    return (lane < 2 * KB && k < count) ? a.val[start + k] : 0.0f;
+    const uint32_t k = position_in(st, 2 * KB, lane);
+    return (lane < 2 * KB && k < (uint32_t)count) ? a.val[start + k] : 0.0f;
   };
   auto issue = [&](int h, int ci) {
     float* yb = stg + h * NB * 256;

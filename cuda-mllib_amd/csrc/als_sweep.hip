@@ -236,7 +236,7 @@ __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WAVES))) void als_rows_kernel(Sweep
       const int64_t u = u0 + __builtin_ctzll(todo);
       const int start = a.row_ptr[u], n = a.row_ptr[u + 1] - start;
       // Shares of whole 32-rating steps.
-      const int share = ((n + 31) / 32 + kRowsWaves - 1) / kRowsWaves * 32;
+      const int share = chunks_of(chunks_of(n, 32), kRowsWaves) * 32;
       const int off = wv * share, cnt = n - off < share ? n - off : share;
       f4 acc[NT];
       if (cnt > 0) {

@@ -3,6 +3,8 @@ rating is covered by exactly one task, tasks run longest first, split rows
 own consecutive partial slots in near-equal chunks, and f > 140 plans whole
 rows."""
 import ctypes as C
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -71,3 +73,34 @@ def test_plan_rejects_decreasing_row_pointers_and_small_buffers():
     assert L.cumf_debug_plan(rp.ctypes.data_as(C.c_void_p), 2, 16, 10, None, 0, C.byref(nt), None, 0,
                              C.byref(nh)) == 1
     assert nt.value == 2 and "too small" in G.last_error()
+
+
+def test_chunk_positions_up_to_int_max_ratings(tmp_path):
+    """The gathers' chunk arithmetic (chunks_of, position_in) against 64-bit
+    integers, for every chunk that a prefetch asks about (up to eight past the
+    end) and every lane of it: a position past the end must never pass for one
+    inside the range."""
+    src = tmp_path / "chunks.cpp"
+    src.write_text(r'''
+#include <climits>
+#include <cstdio>
+#include "als_kernels.h"
+int main() {
+  long bad = 0;
+  for (int64_t edge : {(int64_t)0, (int64_t)INT_MAX - 400})
+    for (int64_t n = edge + 1; n <= edge + 400 && n <= INT_MAX; ++n)
+      for (int size : {8, 16, 32}) {
+        const int nch = cumf::chunks_of((int)n, size);
+        bad += nch != (n + size - 1) / size;
+        for (int64_t ch = nch > 3 ? nch - 3 : 0; ch <= (int64_t)nch + 8; ++ch)
+          for (int lane = 0; lane < size; ++lane)
+            bad += (cumf::position_in((int)ch, size, lane) < (uint32_t)n) != (ch * size + lane < n);
+      }
+  std::printf("%ld\n", bad);
+}
+''')
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    exe = tmp_path / "chunks"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                    f"-I{os.path.dirname(os.path.dirname(os.path.abspath(G.__file__)))}/csrc", str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "0"
