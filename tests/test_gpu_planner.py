@@ -86,3 +86,46 @@ def test_bad_row_pointers_are_refused_and_write_nothing(m, f):
         np.testing.assert_array_equal(X, x0)
     rc, err, X = _device_sweep(rp, ci, cv, theta, m, n, f, 0.05, x0=x0)
     assert rc == 0 and np.all(np.isfinite(X))
+
+
+def _handle_sweep(rp, ci, cv, theta, m, n, f, lam, split):
+    with G.ALS(f, lam, split=split) as h:
+        h.set_ratings(m, n, rp, ci, cv)
+        h.set_factors(theta=theta)
+        h.update_x()
+        return h.get_factors()[0]
+
+
+# Splits below 2,048 come from the caller alone.  Many split rows on both sides
+# of the one-block planner's limit, chunks in the classes of one length (below
+# 256) and in wider ones, one to thousands of chunks a row.
+@pytest.mark.parametrize("split", [1, 7, 96, 256, 300])
+@pytest.mark.parametrize("m", [1, 16384, 16385])
+def test_rows_cut_as_the_callers_split_says(m, split):
+    """The device planner cuts and orders a row's chunks as the host one does,
+    so the factors are the handle's bit for bit."""
+    n, lam, f = 500, 0.05, 8
+    rng = np.random.default_rng(m + split)
+    deg = np.where(rng.random(m) < 0.3, rng.integers(0, 3 * split + 2, m), rng.integers(0, 4, m))
+    deg[rng.integers(0, m, min(m, 4))] = rng.choice([split, split + 1, 2 * split + 1, 70 * split + 3, 20011], min(m, 4))
+    if m == 1:
+        deg[0] = 20011
+    rp, ci, cv = _matrix(deg, n, m)
+    theta = cumf.init_factors(n, f, 3)
+    rc, err, X = _device_sweep(rp, ci, cv, theta, m, n, f, lam, split=split)
+    assert rc == 0, err
+    np.testing.assert_array_equal(X, _handle_sweep(rp, ci, cv, theta, m, n, f, lam, split))
+
+
+@pytest.mark.parametrize("f", [100, 140])
+def test_partial_grams_beyond_the_bound_that_needs_no_wait(f):
+    """Their bound passes 64 MB (28 and 45 KB a chunk), so the host sizes them
+    by the plan's own counts; a smaller call then works in the kept buffers."""
+    n, lam, split = 400, 0.05, 96
+    theta = cumf.init_factors(n, f, 3)
+    for m in (2000, 150):
+        rng = np.random.default_rng(m)
+        rp, ci, cv = _matrix(rng.integers(0, 220, m), n, m)
+        rc, err, X = _device_sweep(rp, ci, cv, theta, m, n, f, lam, split=split)
+        assert rc == 0, err
+        np.testing.assert_array_equal(X, _handle_sweep(rp, ci, cv, theta, m, n, f, lam, split))
