@@ -742,17 +742,24 @@ int run_half_sweep(cumf_handle* h, int side, const Plan& p, const DevBuf& rowp, 
   return CUMF_OK;
 }
 
-// The caller's packed rows go over in one flat copy and are laid out at the
+// The caller's packed rows go over in flat copies and are laid out at the
 // factor stride on the device (and back in download_factors); where the
-// stride is f itself there is nothing to lay out.
+// stride is f itself there is nothing to lay out.  The packed rows pass
+// through h->stage, which cumf_set_ratings sizes (stage_bytes): nothing is
+// allocated here, where hipMalloc and the hipFree before it cost a small
+// call more than its copy.
 int upload_factors(cumf_handle* h, DevBuf& dst, DevBuf& dst_b, const float* src, int64_t rows) {
-  const size_t packed = sizeof(float) * (size_t)rows * h->f;
+  const size_t row = sizeof(float) * (size_t)h->f;
   if (h->ldf == h->f) {
-    CUMF_HIP_TRY(hipMemcpyAsync(dst.p, src, packed, hipMemcpyHostToDevice, h->stream));
+    CUMF_HIP_TRY(hipMemcpyAsync(dst.p, src, row * rows, hipMemcpyHostToDevice, h->stream));
   } else {
-    CUMF_TRY(ensure(h->stage, packed));
-    CUMF_HIP_TRY(hipMemcpyAsync(h->stage.p, src, packed, hipMemcpyHostToDevice, h->stream));
-    CUMF_HIP_TRY(cumf::launch_restride(h->stage.as<float>(), h->f, dst.as<float>(), h->ldf, rows, h->f, h->stream));
+    const int64_t step = (int64_t)(h->stage.bytes / row);
+    for (int64_t r = 0; r < rows; r += step) {
+      const int64_t k = std::min(step, rows - r);
+      CUMF_HIP_TRY(hipMemcpyAsync(h->stage.p, src + r * h->f, row * k, hipMemcpyHostToDevice, h->stream));
+      CUMF_HIP_TRY(cumf::launch_restride(h->stage.as<float>(), h->f, dst.as<float>() + r * h->ldf, h->ldf, k, h->f,
+                                         h->stream));
+    }
   }
   if (h->opt.precision != CUMF_PREC_FP32)
     CUMF_HIP_TRY(cumf::launch_to_bf16(dst.as<float>(), h->ldf, dst_b.p, h->ldb, rows, h->f, h->stream));
@@ -760,15 +767,25 @@ int upload_factors(cumf_handle* h, DevBuf& dst, DevBuf& dst_b, const float* src,
 }
 
 int download_factors(cumf_handle* h, const DevBuf& src, float* dst, int64_t rows) {
-  const size_t packed = sizeof(float) * (size_t)rows * h->f;
-  const void* from = src.p;
-  if (h->ldf != h->f) {
-    CUMF_TRY(ensure(h->stage, packed));
-    CUMF_HIP_TRY(cumf::launch_restride(src.as<float>(), h->ldf, h->stage.as<float>(), h->f, rows, h->f, h->stream));
-    from = h->stage.p;
+  const size_t row = sizeof(float) * (size_t)h->f;
+  if (h->ldf == h->f) {
+    CUMF_HIP_TRY(hipMemcpyAsync(dst, src.p, row * rows, hipMemcpyDeviceToHost, h->stream));
+    return CUMF_OK;
   }
-  CUMF_HIP_TRY(hipMemcpyAsync(dst, from, packed, hipMemcpyDeviceToHost, h->stream));
+  const int64_t step = (int64_t)(h->stage.bytes / row);
+  for (int64_t r = 0; r < rows; r += step) {
+    const int64_t k = std::min(step, rows - r);
+    CUMF_HIP_TRY(cumf::launch_restride(src.as<float>() + r * h->ldf, h->ldf, h->stage.as<float>(), h->f, k, h->f,
+                                       h->stream));
+    CUMF_HIP_TRY(hipMemcpyAsync(dst + r * h->f, h->stage.p, row * k, hipMemcpyDeviceToHost, h->stream));
+  }
   return CUMF_OK;
+}
+
+// What upload_factors and download_factors need for sides of up to `rows`
+// rows: none where the stride is f, else the rows, in pieces of at most 32 MB.
+size_t stage_bytes(const cumf_handle* h, int64_t rows) {
+  return h->ldf == h->f ? 0 : std::min(sizeof(float) * (size_t)rows * h->f, size_t(32) << 20);
 }
 
 }  // namespace
@@ -967,6 +984,7 @@ int cumf_set_ratings(cumf_handle* h, int64_t m, int64_t n, int64_t nnz, const in
   CUMF_TRY(h->cv.alloc(sizeof(float) * nnz));
   CUMF_TRY(h->X.alloc(sizeof(float) * m * h->ldf));
   CUMF_TRY(h->T.alloc(sizeof(float) * n * h->ldf));
+  CUMF_TRY(ensure(h->stage, stage_bytes(h, std::max(m, n))));
   if (h->opt.precision != CUMF_PREC_FP32) {
     CUMF_TRY(h->Xb.alloc(sizeof(uint16_t) * m * h->ldb));
     CUMF_TRY(h->Tb.alloc(sizeof(uint16_t) * n * h->ldb));

@@ -8,6 +8,7 @@ Tolerances (FP32 Gram on MFMA + FP32 Cholesky vs an FP64 oracle):
   * Solution vs oracle: ||x_gpu - x_64|| / ||x_64|| <= 1e-3 per row.
   * Held-out RMSE after full training: |RMSE_gpu - RMSE_64| <= 1e-3.
 """
+import ctypes as C
 import os
 
 import numpy as np
@@ -596,3 +597,33 @@ def test_rows_of_one_rating_at_small_ranks(f):
     want = cv[:, None] * Y / ((Y * Y).sum(1, keepdims=True) + float(np.float32(lam)))
     err = np.linalg.norm(X - want, axis=1) / np.linalg.norm(want, axis=1)
     assert err.max() <= 16 * 2.0 ** -24, err.max()
+
+
+@pytest.mark.parametrize("f", [10, 13])
+def test_factor_transfers_allocate_nothing_and_hold_at_seams(f):
+    """Both directions of a handle whose factor rows are padded on the device
+    (f not a multiple of 4): no device memory is taken after the ratings are
+    set, also for the side that was not uploaded, and rows on both sides of a
+    32 MB piece of the transfer arrive whole and in place."""
+    m, n = 2 * ((32 << 20) // (4 * f)) + 3, 7  # three pieces, the last of three rows
+    rp = np.zeros(m + 1, np.int32)
+    rp[1:] = 1
+    X0 = np.arange(m * f, dtype=np.float32).reshape(m, f) % 8191
+    T0 = cumf.init_factors(n, f, 0)
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert G.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    with G.ALS(f, 0.05) as h:
+        h.set_ratings(m, n, rp, np.zeros(1, np.int32), np.ones(1, np.float32))
+        before = free_bytes()
+        h.set_factors(theta=T0)
+        Xz, T1 = h.get_factors()
+        h.set_factors(X=X0)
+        X1, _ = h.get_factors()
+        assert free_bytes() == before
+    assert np.all(Xz == 0)
+    np.testing.assert_array_equal(T1, T0)
+    np.testing.assert_array_equal(X1, X0)
