@@ -384,11 +384,8 @@ int64_t bf16_stride(int f) {
   return r / 2;
 }
 
-// Register budget of the launches without a tile table: two wavefronts
-// per SIMD while the accumulator tiles leave room for the solver's
-// registers (up to 8 column blocks, f <= 124), one wavefront per SIMD
-// beyond (the two-wavefront build spills several hundred bytes per lane).
-int default_variant(int f) { return cumf::sweep_nb(f) >= 9 ? 1 : 2; }
+// Register budget of the launches without a tile table.
+int default_variant(int f) { return cumf::default_waves(cumf::sweep_nb(f)); }
 
 hipError_t task_launch(const cumf::SweepArgs& a, int variant, hipStream_t s) {
   if (a.solver == CUMF_SOLVER_CG)

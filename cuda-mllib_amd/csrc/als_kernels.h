@@ -144,6 +144,11 @@ hipError_t prepare_compat(int f);
 hipError_t launch_compat(const CompatArgs& a, int64_t nrows, hipStream_t s);
 
 int sweep_nb(int f);
+// Wavefronts per SIMD that the launches without a tile table are built for:
+// two while the accumulator tiles leave room for the solver's registers (up
+// to 8 column blocks, f <= 124), one beyond (the two-wavefront build spills
+// several hundred bytes per lane).
+__host__ __device__ constexpr int default_waves(int NB) { return NB >= 9 ? 1 : 2; }
 size_t partial_floats_per_slot(int f);
 int dump_dim(int f);
 // Clears n <= 64 ints (CG fallback-list length, persistent task counters).

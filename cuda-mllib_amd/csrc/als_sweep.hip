@@ -317,11 +317,15 @@ static hipError_t launch_nb(const SweepArgs& a, hipStream_t s, int which) {
       // wavefront per row where there are fewer, and batches small enough that
       // every group gets one or two of them
       if (bf || a.persistent < 1 || a.ntasks < 1) return hipErrorInvalidValue;
-      const int64_t need = (a.ntasks + kRowsWaves - 1) / kRowsWaves;
-      const int64_t groups = need < a.persistent ? need : a.persistent;
-      const int64_t per = (a.ntasks + 2 * groups - 1) / (2 * groups);
-      const int batch = (int)(per > 64 ? 64 : per);
-      hipLaunchKernelGGL((als_rows_kernel<NB>), dim3((unsigned)groups), dim3(64 * kRowsWaves), 0, s, a, batch);
+      if constexpr (CUMF_TASK_WAVES == default_waves(NB)) {  // the budget its caller takes
+        const int64_t need = (a.ntasks + kRowsWaves - 1) / kRowsWaves;
+        const int64_t groups = need < a.persistent ? need : a.persistent;
+        const int64_t per = (a.ntasks + 2 * groups - 1) / (2 * groups);
+        const int batch = (int)(per > 64 ? 64 : per);
+        hipLaunchKernelGGL((als_rows_kernel<NB>), dim3((unsigned)groups), dim3(64 * kRowsWaves), 0, s, a, batch);
+      } else {
+        return hipErrorInvalidValue;
+      }
     } else
 #endif
     if (which == 3) {

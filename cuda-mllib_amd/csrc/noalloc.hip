@@ -106,7 +106,6 @@ extern "C" int cumf_half_sweep_device_noalloc(hipStream_t stream, const int32_t*
   }
   DeviceScratch ds;
   CUMF_TRY(device_scratch(&ds));
-  const int variant = cumf::sweep_nb(f) >= 9 ? 1 : 2;
   cumf::SweepArgs a{};
   a.row_ptr = d_row_ptr;
   a.col = d_col;
@@ -123,7 +122,7 @@ extern "C" int cumf_half_sweep_device_noalloc(hipStream_t stream, const int32_t*
   a.task_counter = ds.ptr;
   hipLaunchKernelGGL(clear_scratch_kernel, dim3(1), dim3(kScratchInts), 0, stream, ds.ptr);
   CUMF_HIP_TRY(hipGetLastError());
-  CUMF_HIP_TRY(variant == 1 ? cumf::w1::chol::launch_rows_kernel(a, stream)
-                            : cumf::w2::chol::launch_rows_kernel(a, stream));
+  CUMF_HIP_TRY(cumf::default_waves(cumf::sweep_nb(f)) == 1 ? cumf::w1::chol::launch_rows_kernel(a, stream)
+                                                           : cumf::w2::chol::launch_rows_kernel(a, stream));
   return CUMF_OK;
 }
