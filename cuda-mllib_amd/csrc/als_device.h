@@ -396,9 +396,9 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
 // row's column index.  sweep_nb(f) gives 16 (NB-1) <= ldb, so tiles
 // 0 .. NB-2 lie inside the factor row; in the last tile, slots at or past
 // ldb -- and every slot of a row past the end of the range -- come from
-// kZeroRow.  The rating r is then written into columns f and f+1 as bf16(r)
-// and bf16(r - bf16(r)), so b = Y^T r keeps ~16 significant bits (exact for
-// integer ratings).
+// kZeroRow.  The rating r is then written into the columns rc and rc + 1
+// (bf16_rating_col) as bf16(r) and bf16(r - bf16(r)), so b = Y^T r keeps ~16
+// significant bits (exact for integer ratings).
 //
 // MFMA operands come straight from the tiles with ds_read_b64_tr_b16:
 // within a 16-lane group, lane j addresses 4 bf16 of row (8*kg + j/4),
@@ -411,7 +411,7 @@ __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32
 template <int NB>
 __device__ __forceinline__ void gram_range_bf16(f4 (&acc)[num_tiles(NB)], const int32_t* __restrict__ col,
                                                 const float* __restrict__ val,
-                                                const __bf16* __restrict__ theta_b, int64_t ldb, int f,
+                                                const __bf16* __restrict__ theta_b, int64_t ldb, int rc,
                                                 int64_t start, int count, __bf16* __restrict__ lds, int lane) {
   constexpr int TB = KBB * 16;   // bf16 per staged tile
   constexpr int CB = NB * TB;    // bf16 per staged chunk
@@ -423,8 +423,8 @@ __device__ __forceinline__ void gram_range_bf16(f4 (&acc)[num_tiles(NB)], const 
   const int nch = (count + KBB - 1) / KBB;
   // this lane's transpose-read offset inside a tile (bf16 units)
   const int troff = (8 * kg + (j >> 2)) * 16 + 4 * (j & 3);
-  // where the rating halves go: tile and column of f and f+1
-  const int rt0 = (f >> 4) * TB + (f & 15), rt1 = ((f + 1) >> 4) * TB + ((f + 1) & 15);
+  // where the rating halves go
+  const int rt0 = (rc >> 4) * TB + (rc & 15), rt1 = ((rc + 1) >> 4) * TB + ((rc + 1) & 15);
 
   auto load_ci = [&](int ch) -> int {
     const int k = ch * KBB + sr;
@@ -1623,8 +1623,8 @@ template <int NB, bool BF>
 __device__ __forceinline__ void gram_any(f4 (&acc)[num_tiles(NB)], const SweepArgs& a, int64_t start, int count,
                                          float* lds, int lane) {
   if constexpr (BF)
-    gram_range_bf16<NB>(acc, a.col, a.val, reinterpret_cast<const __bf16*>(a.theta_b), a.ldb, a.f,
-                        start, count, reinterpret_cast<__bf16*>(lds), lane);
+    gram_range_bf16<NB>(acc, a.col, a.val, reinterpret_cast<const __bf16*>(a.theta_b), a.ldb,
+                        bf16_rating_col(a.f, NB), start, count, reinterpret_cast<__bf16*>(lds), lane);
   else
     gram_range<NB>(acc, a.col, a.val, a.theta, a.ldf, start, count, lds, lane);
 }
@@ -1637,8 +1637,8 @@ __device__ __forceinline__ void solve_row(f4 (&acc)[num_tiles(NB)], const SweepA
                                           int64_t row, __bf16* xb, int lane, int entry,
                                           const float* xpre = nullptr) {
   float* xrow = a.x + row * a.ldf;
-  const int bcol = bf ? a.f : (int)a.ldf;
-  const int bcol2 = bf ? a.f + 1 : -1;
+  const int bcol = bf ? bf16_rating_col(a.f, NB) : (int)a.ldf;
+  const int bcol2 = bf ? bcol + 1 : -1;
   if constexpr (CG) {
     const CgParams cp{a.cg_iters, a.cg_rounds, a.cg_tol, a.warm};
     const float* x0row = a.x0 ? a.x0 + row * a.ldf : nullptr;

@@ -144,6 +144,11 @@ hipError_t prepare_compat(int f);
 hipError_t launch_compat(const CompatArgs& a, int64_t nrows, hipStream_t s);
 
 int sweep_nb(int f);
+// First of the two columns (high and low part) that the rating takes in the
+// BF16 layout of NB column blocks: f, or the last block's first column where f
+// lies before that block (f % 16 above 12): the solves read the right-hand
+// side from the last block.
+__host__ __device__ constexpr int bf16_rating_col(int f, int NB) { return f > 16 * (NB - 1) ? f : 16 * (NB - 1); }
 // Wavefronts per SIMD that the launches without a tile table are built for:
 // two while the accumulator tiles leave room for the solver's registers (up
 // to 8 column blocks, f <= 124), one beyond (the two-wavefront build spills

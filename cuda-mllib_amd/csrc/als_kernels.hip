@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void copy_kernel(const f4* __restrict__ src, f
 // ---------------------------------------------------------------------------
 // 16-column blocks of the augmented tile grid: room for the FP32 layout
 // (factor columns to ldf, rating at ldf) and the BF16 layout (factor
-// columns to ldb = round_up(f,8), rating hi/lo at f, f+1).
+// columns to ldb = round_up(f,8), rating hi/lo from bf16_rating_col on).
 int sweep_nb(int f) {
   const int ldf = (f + 3) & ~3, ldb = (f + 7) & ~7;
   int w = ldf + 1;

@@ -295,7 +295,9 @@ int cumf_autotune(cumf_handle* h, int reps, const char* path);
 /* Augmented Gram of the listed rows of the X side (side 0, over the CSR)
  * or Theta side (side 1, over the CSC), ridge included, as dense D x D
  * row-major FP32 (D = cumf_debug_gram_dim(f)); A is the leading f x f
- * block, b sits in column round_up(f,4).  out: host, nrows * D * D. */
+ * block, b sits in column round_up(f,4); with CUMF_PREC_BF16_GRAM it is the
+ * sum of two columns, f and f + 1, or the next multiple of 16 and the column
+ * after it where f % 16 > 12.  out: host, nrows * D * D. */
 int cumf_debug_gram_dim(int f);
 int cumf_debug_row_gram(cumf_handle* h, int side, const int32_t* rows, int64_t nrows, float* out);
 /* The host task planner alone (no device): the wavefront tasks of a CSR

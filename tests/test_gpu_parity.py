@@ -627,3 +627,35 @@ def test_factor_transfers_allocate_nothing_and_hold_at_seams(f):
     assert np.all(Xz == 0)
     np.testing.assert_array_equal(T1, T0)
     np.testing.assert_array_equal(X1, X0)
+
+
+@pytest.mark.parametrize("f", [12, 13, 14, 15, 16, 29, 30, 31, 45, 46, 47, 61, 62, 63, 77, 78, 79, 93, 94, 95, 109, 110,
+                               111, 125, 126, 127, 128])
+@pytest.mark.parametrize("solver", [G.CUMF_SOLVER_CHOLESKY, G.CUMF_SOLVER_CG])
+def test_bf16_ranks_up_to_a_block_edge(f, solver):
+    """BF16 Gram at ranks whose factor columns end one to three columns before
+    a 16-column block does: the rating's columns then lie in the block after
+    it.  Rows with and without a split; each one's residual against the FP64
+    system on the BF16 factors is at most 1e-5 (Cholesky; CG: twice its
+    tolerance of 1e-5), as at every other rank."""
+    lam, n = 0.05, 900
+    rng = np.random.default_rng(f)
+    counts = np.array([1, 2, 15, 16, 31, 32, 33, 64, 95, 96, 97, 128, 200, 256, 257, 600, 899])
+    m = counts.shape[0]
+    rp = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    ci = np.concatenate([rng.choice(n, c, replace=False) for c in counts]).astype(np.int32)
+    cv = rng.integers(1, 6, rp[-1]).astype(np.float32)
+    T = cumf.init_factors(n, f, 5)
+    with G.ALS(f, lam, precision=G.CUMF_PREC_BF16_GRAM, solver=solver, split=256) as h:
+        h.set_ratings(m, n, rp, ci, cv)
+        h.set_factors(theta=T)
+        h.update_x()
+        X, _ = h.get_factors()
+        assert h.stats()["failed_rows"] == 0
+    Tr = _bf16(T)
+    for u, cnt in enumerate(counts):
+        Y = Tr[ci[rp[u]:rp[u + 1]]].astype(np.float64)
+        b = Y.T @ cv[rp[u]:rp[u + 1]].astype(np.float64)
+        x = X[u].astype(np.float64)
+        res = np.linalg.norm(b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(cnt)) * x) / np.linalg.norm(b)
+        assert res <= (1e-5 if solver == G.CUMF_SOLVER_CHOLESKY else 2e-5), (f, cnt, res)
