@@ -206,12 +206,11 @@ struct DevicePlan {
 // Longest task of a matrix of nnz ratings: the caller's split size, less
 // where that would leave the chip waiting for one wavefront.  A task is at
 // most half of a wavefront's share when 2,048 of them (two per SIMD) run side
-// by side, and never under 2,048 ratings (the entry point that cannot split
-// solves rows up to that length whole, with the same result).  Measured at 60,023 x 17,770, 12.4 million ratings, f = 50: the task
-// kernel 1.45 ms with a 16,384-rating task at its head; the whole call 0.85 ms
-// with 3,023.
+// by side, and never under kWholeRowMax ratings.  Measured at 60,023 x 17,770,
+// 12.4 million ratings, f = 50: the task kernel 1.45 ms with a 16,384-rating
+// task at its head; the whole call 0.85 ms with 3,023.
 int adaptive_split(int split, int64_t nnz) {
-  return (int)std::min<int64_t>(split, std::max<int64_t>(2048, nnz / 4096));
+  return (int)std::min<int64_t>(split, std::max<int64_t>(cumf::kWholeRowMax, nnz / 4096));
 }
 
 int check_f(int f) {
@@ -2128,7 +2127,7 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
       return CUMF_ERR_INVALID;
     }
     CUMF_TRY(check_f(f));
-    // The factor buffers and the task plan come from the device's cache
+    // The factor buffers and the plan's come from the device's cache
     // when it is free (see SweepCache), else from allocations of this call.
     CacheLease lease;
     DevBuf local_theta, local_x;

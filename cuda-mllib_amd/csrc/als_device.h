@@ -11,9 +11,9 @@
 // One 64-lane wavefront per task (a row, or a chunk of a long row):
 //   * Gram: the factor rows of each chunk of ratings are gathered into LDS
 //     and the augmented Gram [Y r]^T [Y r] is accumulated on MFMA over the
-//     NB(NB+1)/2 upper 16x16 tiles (FP32: v_mfma_f32_16x16x4_f32; BF16:
-//     v_mfma_f32_16x16x32_bf16 with the rating split into a BF16 high and
-//     low column).  The extra column(s) carry b = Y^T r.
+//     NB(NB+1)/2 upper 16x16 tiles with v_mfma_f32_16x16x32_bf16 (FP32: six
+//     products of three-way split floats; BF16: one, with the rating split
+//     into a BF16 high and low column).  The extra column(s) carry b = Y^T r.
 //   * The accumulators stay in registers (lane l holds rows
 //     16I + 4(l/16) + {0..3} of column 16J + l%16 of tile (I, J)), and a
 //     blocked right-looking Cholesky runs on the tiles in place: per
@@ -165,7 +165,10 @@ static __device__ const float kZeroRow[256] = {};
 // operands; a product rounded to FP32 is off by at most 2^-24).  A sum gains
 // more than that from fewer roundings (split_tiles).  Rounding h instead would
 // leave out at most 2^-24, for 1 to 7% of every FP32 half-sweep, and moved no
-// error of a whole row above one block.  Six v_mfma_f32_16x16x32_bf16 (16
+// error of a whole row above one block.  The matrix pipe takes parts below
+// 2^-126 as zero, so factors below about 1e-33 keep fewer bits: a row with
+// nothing larger is off by 4e-6 at 1e-35 and 3e-4 at 1e-37 where plain FP32
+// products stay at 2e-7.  Six v_mfma_f32_16x16x32_bf16 (16
 // cycles of the matrix pipe each) do 32 k-values where eight
 // v_mfma_f32_16x16x4_f32 take 32 cycles each.
 // ---------------------------------------------------------------------------
@@ -278,9 +281,11 @@ __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmc
 // are 168 matrix instructions of 16 cycles beside 308 VALU instructions of the
 // split, 112 additions and 56 LDS reads, against 224 matrix instructions of 32
 // cycles for plain FP32 ones.  Measured at 480,189 x 17,770, 99 million
-// ratings, f = 100, whole half-sweeps: Theta 13.7 -> 7.4 ms (40 GB of gathers,
-// 5.4 TB/s: now bound by them), X 16.5 -> 11.3 ms (now bound by its solves);
-// error against 64 bits 4.9e-6 -> 1.0e-6 and 1.2e-6 -> 5.4e-7.
+// ratings, f = 100, whole half-sweeps: Theta 13.7 -> 7.4 ms, X 16.5 -> 11.3 ms
+// (7.0 and 10.0 ms with what came later); error against 64 bits 4.9e-6 ->
+// 1.0e-6 and 1.2e-6 -> 5.4e-7.  In the Theta launch a SIMD's matrix pipe is
+// busy for 66% and its VALU for 67% of the cycles, at 1.7 GHz under that load,
+// and 33 of the 40 GB of gathers come from beyond L2 (4.4 TB/s).
 // ---------------------------------------------------------------------------
 template <int NB>
 __device__ __forceinline__ void gram_range(f4 (&acc)[num_tiles(NB)], const int32_t* __restrict__ col,

@@ -92,6 +92,12 @@ struct SweepArgs {
 __host__ __device__ constexpr int chunks_of(int count, int size) { return (count - 1) / size + 1; }
 __host__ __device__ constexpr uint32_t position_in(int ch, int size, int i) { return (uint32_t)ch * size + i; }
 
+// Rows up to this length are solved whole, whatever the matrix: the finest cut
+// that adaptive_split makes by itself, and the longest row that one wavefront
+// of launch_rows_kernel solves.  One constant, so that both give the same
+// factors up to it; the value is not a measured optimum.
+constexpr int kWholeRowMax = 2048;
+
 // Longest row the dual form takes (three staged chunks of 32 ratings).
 constexpr int kDualMaxRatingsHost = 95;
 

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void to_bf16_kernel(const float* __restrict__ 
 // Rows of `cols` floats from stride lds to stride ldd, the columns past
 // `cols` written as zero (factors between the caller's packed layout and the
 // padded rows the sweeps read).  One pass at copy speed: a block takes whole
-// rows of about 8,192 destination floats, so the index division is 32 bits
+// rows of about 1,024 destination floats, so the index division is 32 bits
 // wide.  It stands in for hipMemcpy2D, which moves pageable host memory row
 // by row (12,000 rows of 128 bytes: 20 ms up and 85 ms down; one flat copy
 // and this kernel: 0.1 ms) and for device rows needed a fill before it.

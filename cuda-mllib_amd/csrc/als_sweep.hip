@@ -203,17 +203,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
 #if CUMF_SWEEP_SOLVER == 0
 // The rows 0 .. ntasks themselves, FP32, without a task list, plan or scratch
 // memory: one work-group per CU, two passes.
-//   * Rows of more than kLongRow ratings are solved by the work-group
+//   * Rows of more than kWholeRowMax ratings are solved by the work-group
 //     together: each wavefront forms the Gram of its share of the ratings, the
 //     shares are added through LDS in wavefront order, and wavefront 0 solves.
 //     The groups take batches of rows from a counter to look for them.  By
 //     itself a wavefront needs 0.84 ms for a row of 15,136 ratings at f = 64,
 //     which was all of a 2,048-row call; the call now takes 0.19 ms.
 //   * The other rows go to the wavefronts one by one, from a second counter,
-//     solved as the task kernel solves them (the device entry points with a
-//     plan do not split rows up to kLongRow ratings either).
+//     solved as the task kernel solves them (with the default split size the
+//     entry points with a plan do not cut them either).
 constexpr int kRowsWaves = 4 * CUMF_TASK_WAVES;  // wavefronts per group: all a CU holds
-constexpr int kLongRow = 2048;
 
 template <int NB>
 __global__ __launch_bounds__(64 * kRowsWaves)
@@ -231,7 +230,7 @@ __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WAVES))) void als_rows_kernel(Sweep
     const int64_t u0 = b * batch;
     if (u0 >= a.ntasks) break;
     const int64_t mine = u0 + lane;
-    const bool is_long = lane < batch && mine < a.ntasks && a.row_ptr[mine + 1] - a.row_ptr[mine] > kLongRow;
+    const bool is_long = lane < batch && mine < a.ntasks && a.row_ptr[mine + 1] - a.row_ptr[mine] > kWholeRowMax;
     for (uint64_t todo = __ballot(is_long); todo; todo &= todo - 1) {
       const int64_t u = u0 + __builtin_ctzll(todo);
       const int start = a.row_ptr[u], n = a.row_ptr[u + 1] - start;
@@ -274,7 +273,7 @@ __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WAVES))) void als_rows_kernel(Sweep
   for (int64_t idx = (int64_t)blockIdx.x * kRowsWaves + wv; idx < a.ntasks;) {
     lds_order();
     const int start = a.row_ptr[idx], n = a.row_ptr[idx + 1] - start;
-    if (n <= kLongRow) run_task<NB, false, false>(a, Task{(int32_t)idx, start, n, -1}, lds, lane);
+    if (n <= kWholeRowMax) run_task<NB, false, false>(a, Task{(int32_t)idx, start, n, -1}, lds, lane);
     if (waves >= a.ntasks) break;  // (every row had its wavefront)
     int more = 0;
     if (lane == 0) more = atomicAdd(a.task_counter, 1);

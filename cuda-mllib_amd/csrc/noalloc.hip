@@ -1,10 +1,10 @@
 // noalloc.hip -- a half-sweep entry point that allocates nothing.
 //
-// cumf_half_sweep_device allocates its task plan, partial-Gram scratch and
-// counters and reads the row pointers back to plan.  Callers that cannot
-// allocate or synchronise (code under HIP graph capture, tight serving
+// cumf_half_sweep_device grows its task plan, partial-Gram scratch and
+// counters to the largest call so far and waits for its stream.  Callers that
+// cannot allocate or synchronise (code under HIP graph capture, tight serving
 // loops) use cumf_half_sweep_device_noalloc instead: same arithmetic (FP32
-// Gram on MFMA, FP32 Cholesky), no host work beyond argument checks, no
+// Gram from split products, FP32 Cholesky), no host work beyond argument checks, no
 // device allocation and no synchronisation.  One work-group per CU takes
 // whole rows from counters (long rows together, the others wavefront by
 // wavefront); the counters and the failed-row count live in `scratch`, a

@@ -71,7 +71,10 @@ void doALSWithCSR(hipStream_t cuda_stream, int* csrRowIndex, int* csrColIndex, f
 
 #define CUMF_OPTIONS_VERSION 1
 
-#define CUMF_PREC_FP32 0        /* FP32 Gram (split BF16 products), FP32 Cholesky */
+#define CUMF_PREC_FP32 0        /* FP32 Gram (split BF16 products), FP32 Cholesky.
+                                   Factors below about 1e-33 keep fewer bits: a
+                                   row with nothing larger is off by 4e-6 at
+                                   1e-35, 3e-4 at 1e-37 */
 #define CUMF_PREC_BF16_GRAM 1   /* Gram on BF16 MFMA (FP32 accumulation) from BF16
                                    copies of the factors, b from a BF16 hi/lo split
                                    of the ratings, FP32 Cholesky */
@@ -211,8 +214,10 @@ int cumf_half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const i
  * but: no device allocation, no host readback and no synchronisation (the
  * work is enqueued on `stream`); whole rows taken from counters by one
  * work-group per CU (a row of more than 2,048 ratings by the group
- * together); the CSR must be consistent (row_ptr[0] = 0, row_ptr[m] = nnz, columns < n),
- * which is not checked on the host.  Limits: f a multiple of 4 in [4, 140]
+ * together).  A group holds 40 to 139 KB of its CU's 160 KB of LDS (by f), so
+ * beside other kernels the call waits for CUs with that much left.  The CSR
+ * must be consistent (row_ptr[0] = 0, row_ptr[m] = nnz, columns < n), which is
+ * not checked on the host.  Limits: f a multiple of 4 in [4, 140]
  * (factor rows are read in place, row stride f), m <= INT_MAX - 2^20.  Its
  * only scratch memory is a 256-byte device array per GPU (the row counters
  * and the failed-row count), held until the process ends and shared by

@@ -202,3 +202,10 @@ def test_rows_at_every_step_and_block_edge(f):
         x = X[u].astype(np.float64)
         res = b - Y.T @ (Y @ x) - float(np.float32(lam) * np.float32(cnt)) * x
         assert np.linalg.norm(res) <= 1e-5 * np.linalg.norm(b), (f, cnt, np.linalg.norm(res) / np.linalg.norm(b))
+
+
+# The block counts that the ranks above leave out, 12 and 14, and the primal
+# kernel's line between one operand buffer (f <= 220) and two.
+@pytest.mark.parametrize("f", [173, 188, 205, 220, 221])
+def test_rows_at_every_step_and_block_edge_at_the_other_block_counts(f):
+    test_rows_at_every_step_and_block_edge(f)
