@@ -191,7 +191,8 @@ struct Plan {
 
 // A plan made on the device for one call of the device entry points: the
 // buffers it works in are kept (at their largest so far) in the device's
-// cache and reused by the next call.
+// cache and reused by the next call, the partial Grams' up to a bound
+// (ensure_partial).
 struct DevicePlan {
   DevBuf tasks, heavy, partial, work;
   cumf::PlanSummary* summary = nullptr;  // pinned host memory the planner writes
@@ -1964,6 +1965,14 @@ struct SyncOnFailure {
   void done() { armed = false; }
 };
 
+// Room for a call's partial Grams in the kept buffer.  A caller's small split
+// size can make them many gigabytes, which would stay for the life of the
+// process: beyond 1 GB a buffer over four times what the call needs is given
+// back for one that fits.
+int ensure_partial(DevBuf& b, size_t bytes) {
+  return b.bytes > (size_t(1) << 30) && b.bytes / 4 > bytes ? b.alloc(bytes) : ensure(b, bytes);
+}
+
 // Where the bound on a matrix's partial Grams is at most this, they are sized
 // by the bound and the sweep is launched behind the planner without waiting
 // for it; above it the host waits for the plan's counts (about 15 us).
@@ -2047,7 +2056,7 @@ int half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_
     nheavy = plan.summary->nheavy;
     nslots = plan.summary->nslots;
   }
-  if (!o.compat_hermitian_bug) CUMF_TRY(ensure(plan.partial, slot_bytes * (size_t)nslots));
+  if (!o.compat_hermitian_bug) CUMF_TRY(ensure_partial(plan.partial, slot_bytes * (size_t)nslots));
   const float* theta = d_theta;
   float* x = d_x;
   if (ldf != f) {

@@ -202,7 +202,8 @@ const char* cumf_last_error(void);
 /* Device-resident half-sweep with caller-owned device buffers (nothing
  * consumed, nothing copied): x (m x f) from theta (n x f) over the CSR.
  * The tasks are planned on the device from the row pointers.  The workspace
- * is kept per GPU between calls (at its largest so far), and the call
+ * is kept per GPU between calls (at its largest so far; the partial Grams of
+ * split rows go back when over 1 GB and four times what a call needs), and the call
  * synchronises `stream` before returning; calls that overlap on one GPU
  * work with buffers of their own. */
 int cumf_half_sweep_device(hipStream_t stream, const int32_t* d_row_ptr, const int32_t* d_col,

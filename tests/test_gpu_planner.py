@@ -129,3 +129,28 @@ def test_partial_grams_beyond_the_bound_that_needs_no_wait(f):
         rc, err, X = _device_sweep(rp, ci, cv, theta, m, n, f, lam, split=split)
         assert rc == 0, err
         np.testing.assert_array_equal(X, _handle_sweep(rp, ci, cv, theta, m, n, f, lam, split))
+
+
+def test_large_partial_grams_are_given_back():
+    """A small split size makes 1.4 GB of partial Grams (f = 140, 45 KB a
+    chunk); the next ordinary call gives them back and is right."""
+    n, lam, f = 400, 0.05, 140
+    theta = cumf.init_factors(n, f, 3)
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert G.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    rng = np.random.default_rng(0)
+    small, big = _matrix(rng.integers(0, 220, 50), n, 50), _matrix(np.full(2100, 100), n, 2100)
+    rc, err, X0 = _device_sweep(*small, theta, 50, n, f, lam, split=96)
+    assert rc == 0, err
+    before = free_bytes()
+    rc, err, _ = _device_sweep(*big, theta, 2100, n, f, lam, split=7)
+    assert rc == 0, err
+    assert before - free_bytes() > 1 << 30
+    rc, err, X1 = _device_sweep(*small, theta, 50, n, f, lam, split=96)
+    assert rc == 0, err
+    assert before - free_bytes() < 64 << 20
+    np.testing.assert_array_equal(X1, X0)
