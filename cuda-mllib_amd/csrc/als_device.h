@@ -2075,9 +2075,8 @@ __host__ __device__ constexpr int fp32_dual_max_blocks(int NB) { return NB > 7 ?
 // ratings: 446 -> 419 .. 433 us at f = 12.
 __host__ __device__ constexpr int fp32_dual_max_ratings(int NB) { return NB > 1 ? 16 * fp32_dual_max_blocks(NB) - 1 : 4; }
 
-// Whether the kernels of NB blocks solve a whole FP32 row of n ratings in the
-// dual form.  Besides the line above, and unless the launch is a tile table's
-// Cholesky one:
+// Longest whole FP32 row that a launch of NB blocks solves in the dual form.
+// Besides the line above, and unless the launch is a tile table's Cholesky one:
 //   * a ridge: without one the f x f system of so short a row is singular and
 //     the row fails; its n x n one need not be;
 //   * n <= f (in the last block column f may be up to 3 below n): Y Y^T has
@@ -2085,9 +2084,11 @@ __host__ __device__ constexpr int fp32_dual_max_ratings(int NB) { return NB > 1 
 //     being singular, where Y^T Y needs none.  Errors against 64 bits at
 //     f = 13, 14 ratings a row: 2e-4 against 4e-5 at lambda = 1e-5, 2e-2
 //     against 6e-5 at 1e-7, and failed rows below that.
-template <int NB>
-__device__ __forceinline__ bool fp32_takes_dual(const SweepArgs& a, int n) {
-  return !a.primal && a.lambda > 0.0f && n <= fp32_dual_max_ratings(NB) && n <= a.f;
+// One number for the launch: the three tests on the device cost the smallest
+// call (600 rows) 0.4 us.
+inline int fp32_dual_limit(const SweepArgs& a, int NB) {
+  if (a.precision != 0 || a.primal || !(a.lambda > 0.0f)) return 0;
+  return fp32_dual_max_ratings(NB) < a.f ? fp32_dual_max_ratings(NB) : a.f;
 }
 
 }  // namespace cumf

@@ -68,6 +68,9 @@ struct SweepArgs {
   // != 0: FP32 rows in the f x f system whatever their length (a tile table's
   // Cholesky); 0: short ones in the dual form.
   int primal;
+  // Longest whole FP32 row that the launch solves in the dual form (0: none);
+  // the launchers set it (fp32_dual_limit).
+  int dual_limit;
   // persistent > 0: launch that many wavefronts, each taking tasks from
   // *task_counter (zero before the launch) until ntasks are taken.
   // launch_rows_kernel: that many work-groups over the rows 0 .. ntasks of

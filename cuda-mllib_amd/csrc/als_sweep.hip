@@ -65,7 +65,7 @@ __device__ __forceinline__ void run_task(const SweepArgs& a, const Task& t, floa
   }
 
   if constexpr (!BF && !CG) {
-    if (t.slot < 0 && fp32_takes_dual<NB>(a, t.count)) {
+    if (t.slot < 0 && t.count <= a.dual_limit) {
       fp32_dual_row<fp32_dual_max_blocks(NB)>(a, t, lds, lane);
       return;
     }
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WA
       const int cnt = a.row_ptr[row + 1] - a.row_ptr[row];
       lds_order();
       if constexpr (!BF) {  // as the task kernel solves them
-        if (cnt > 0 && fp32_takes_dual<NB>(a, cnt)) {
+        if (cnt > 0 && cnt <= a.dual_limit) {
           fp32_dual_row<fp32_dual_max_blocks(NB)>(a, Task{(int32_t)row, (int32_t)s, cnt, -1}, lds, lane);
           continue;
         }
@@ -285,7 +285,9 @@ __attribute__((amdgpu_waves_per_eu(CUMF_TASK_WAVES))) void als_rows_kernel(Sweep
 constexpr int kFallbackGrid = 2048;  // work-groups walking the fallback list
 
 template <int NB>
-static hipError_t launch_nb(const SweepArgs& a, hipStream_t s, int which) {
+static hipError_t launch_nb(const SweepArgs& args, hipStream_t s, int which) {
+  SweepArgs a = args;
+  a.dual_limit = fp32_dual_limit(args, NB);
   constexpr bool CG = CUMF_SWEEP_SOLVER == 1;
   const bool bf = a.precision != 0;
   size_t shmem = sizeof(float) * (size_t)cmax(lds_floats_nb(NB, bf), CG ? cg_lds_floats(NB, a.f) : 0);
